@@ -586,7 +586,7 @@ def prefill_eval_bench(args):
         "dtype": "fp16 inputs, fp32 scores and products", "data": "synthetic",
         "config": {"workload": c["workload"], "global_batch": 1, "seq_len": T, "parallelism": "single-gpu",
                    "base": "uniform INT3 g=32 quant-dequant (K_hat, V_hat)", "kind": "both, output_aware V score"},
-        "roofline": {"bound": "mfma", "kernel": "prefill_eval_kernel<64>", "achieved": round(tflops, 3),
+        "roofline": {"bound": "mfma", "kernel": "prefill_eval_kernel<64, 16>", "achieved": round(tflops, 3),
                      "peak": 157.3, "unit": "TFLOP/s", "frac": round(tflops / 157.3, 4), "traffic": None,
                      "algorithmic_flops_per_launch": flops, "launch_us": round(ms * 1e3, 2),
                      "note": "fp32 arithmetic against the fp32 peak"},
