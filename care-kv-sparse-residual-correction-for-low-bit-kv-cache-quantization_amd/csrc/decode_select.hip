@@ -22,7 +22,7 @@
 #include <type_traits>
 
 #include "block_util.h"
-#include "decode_common.h"
+#include "decode_page.h"
 #include "host_util.h"
 
 namespace carekv {
@@ -676,20 +676,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
   for (int i = sel_run + tid; i < a.diag_cap; i += kBlock) diagp[i] = -1;
 }
 
-// Wave-per-query form of decode_select_kernel<D, false, true> for rows of
+// Wave-per-query form of decode_select_kernel<D, false, K1> for rows of
 // at most 256 pages (prompt rows of the prefill correction, short decode
 // rows): one wave per query column, four columns per work-group and no
 // barrier, where the work-group form spends most of a short row on its
-// block reductions and four radix passes.  Lane l holds pages l + 64j.
-// Every float sum is taken in the work-group form's order (a butterfly per
-// 64 pages, then the four totals in page order), the k-th largest key comes
-// from a binary search over its 31 bits, and ties at it are taken in
-// candidate order, so the (M, L), masks and diag lists are the same bits.
-// One K and one V candidate per page (k_cap = v_cap = 1), the joint or
-// separate policy, no adaptive_score, correction on, the moments' K score.
-template <int D>
+// block reductions and four radix passes.  Lane l holds pages l + 64j, with
+// one K and one V candidate each (K1) or up to k_cap and v_cap of them.
+// Every float sum is taken in the work-group form's order (a page's slots in
+// rank order, a butterfly per 64 pages, then the four totals in page order),
+// the k-th largest key comes from a binary search over its 31 bits, and ties
+// at it are taken in candidate order, so the (M, L), masks and diag lists are
+// the same bits.  The search ends as soon as exactly k keys lie above its
+// bound (usually after half the bits) and starts at the largest key's top bit.
+// The joint or separate policy, no adaptive_score, correction on, the moments'
+// K score.
+template <int D, bool K1>
 __global__ __launch_bounds__(256) void decode_select_wave_kernel(carekv_arena A, DecodeArgs a) {
   constexpr int NCG = D / 32;
+  constexpr int KC = K1 ? 1 : NCG, VC = K1 ? 1 : kVtb;  // candidates a lane holds per page
   constexpr int NJ = 4;  // pages per lane
   const int GQ = a.GQ, ngq = (GQ + 3) / 4;
   const int lane = threadIdx.x & 63;
@@ -752,35 +756,40 @@ __global__ __launch_bounds__(256) void decode_select_wave_kernel(carekv_arena A,
   const float L = ordered_sum(lj, (nsr + 63) / 64);
   if (lane == 0) { a.ml[bq * 2] = M; a.ml[bq * 2 + 1] = L; }
 
-  // ---- one K and one V score per page (decode_select_kernel's K1 scoring)
-  const float* recq = a.rec + bq * a.Pmax * a.F;
+  // ---- the page's candidate scores (decode_select_kernel's scoring)
+  const int k_cap = K1 ? 1 : a.k_cap, v_cap = K1 ? 1 : a.v_cap, F = K1 ? 7 : a.F;
+  const float* recq = a.rec + bq * a.Pmax * F;
   const float invL = L > 0.f ? (a.pf ? 1.f : 1.f / L) : 0.f;
   const float* vsq_row = a.pf ? a.pf_vsq + (long)kvh * a.pf_pages : nullptr;
   const bool sens1 = a.sens_d == 1.0;
-  float sK[NJ], sV[NJ];
-  int cgK[NJ], vbV[NJ];
+  float sK[KC][NJ], sV[VC][NJ];
+  int subK[NJ], subV[NJ];  // the candidates' channel groups / V blocks, 4 bits each
   int cntK = 0, cntV = 0;
   bool ovf = false;
-  // Two page slices at a time: the loads of both are issued (every lane,
-  // its page clamped to the row's last) before either is scored, so that a
-  // lane waits one memory round trip per pair of slices, not per slice; the
-  // scoring is the same arithmetic on the same values.
   struct PageIn {
     int nv, hm, ksl[NCG], vsl[kVtb];
-    float vsq, r[7];
+    float vsq, r[K1 ? 7 : 2 + 4 * NCG + kVtb];
     uint2 e2;
   };
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
-    sK[j] = sV[j] = -1.f;
-    cgK[j] = vbV[j] = -1;
+#pragma unroll
+    for (int r = 0; r < KC; ++r) sK[r][j] = -1.f;
+#pragma unroll
+    for (int r = 0; r < VC; ++r) sV[r][j] = -1.f;
+    subK[j] = subV[j] = 0;
   }
+  // K1: two page slices at a time, the loads of both issued (every lane,
+  // its page clamped to the row's last) before either is scored, so that a
+  // lane waits one memory round trip per pair of slices, not per slice; the
+  // scoring is the same arithmetic on the same values.
+  constexpr int NH = K1 ? 2 : 1;
 #pragma unroll
-  for (int j0 = 0; j0 < NJ; j0 += 2) {
+  for (int j0 = 0; j0 < NJ; j0 += NH) {
     if (j0 >= njp) break;
-    PageIn in[2];
+    PageIn in[NH];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < NH; ++h) {
       const int pc = min(lane + 64 * (j0 + h), np - 1);
       const long pg = pg_base + pc;
       in[h].nv = A.valid[pg];
@@ -789,12 +798,12 @@ __global__ __launch_bounds__(256) void decode_select_wave_kernel(carekv_arena A,
       load_slots<NCG>(in[h].ksl, A.k_slot + pg * NCG);
       load_slots<kVtb>(in[h].vsl, A.v_slot + pg * kVtb);
       in[h].e2 = *reinterpret_cast<const uint2*>(A.v_err + pg * kVtb);
-      const float* rp = recq + (long)pc * 7;
+      const float* rp = recq + (long)pc * F;
 #pragma unroll
-      for (int k = 0; k < 7; ++k) in[h].r[k] = rp[k];
+      for (int k = 0; k < (K1 ? 7 : 2 + 4 * NCG + kVtb); ++k) in[h].r[k] = K1 || k < F ? rp[k] : 0.f;
     }
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < NH; ++h) {
       const int j = j0 + h;
       const int p = lane + 64 * j;
       if (p >= np) continue;
@@ -803,34 +812,85 @@ __global__ __launch_bounds__(256) void decode_select_wave_kernel(carekv_arena A,
       const int* ksl = in[h].ksl;
       const int* vsl = in[h].vsl;
       const uint2 e2 = in[h].e2;
-      const float r0 = in[h].r[0], M2 = in[h].r[1], M3 = in[h].r[2], M4 = in[h].r[3], Ds = in[h].r[4],
-                  es = in[h].r[5], E = in[h].r[6];
+      const float* rec = in[h].r;
       const bool ok = L > 0.f && nv > 0 && hm;
-      const float c = ok ? exp2_dn(r0 - M) * invL : 0.f;
-      int nks = 0, nvs = 0, cg1 = -1, vb1 = -1;
-#pragma unroll
-      for (int cg = NCG - 1; cg >= 0; --cg)
-        if (slot_ok(A, ksl[cg])) { ++nks; cg1 = cg; }
-#pragma unroll
-      for (int vb = kVtb - 1; vb >= 0; --vb)
-        if (slot_ok(A, vsl[vb])) { ++nvs; vb1 = vb; }
-      ovf |= hm && (nks > 1 || nvs > 1);
-      cgK[j] = cg1;
-      vbV[j] = vb1;
-      if (ok && nks > 0) {
+      const float c = ok ? exp2_dn(rec[0] - M) * invL : 0.f;
+      auto kscore = [&](float M2, float M3, float M4, float Ds, float es, float vnorm) {
         const float wr = es * (1.f - c * es);
         const float q2 = (M2 - c * (2.f * M3 - c * M4)) + Ds * (wr * wr);
-        float ks = kscore_underflows(c, M2, Ds, es) ? 0.f : (c * sqrt_dn(fmaxf(q2, 0.f))) * __builtin_amdgcn_sqrtf(vsq);
-        if (!isfinite(ks)) ks = 0.f;
-        sK[j] = ks * a.sens;
-        ++cntK;
-      }
-      if (ok && vb1 >= 0 && vb1 * kVtb < nv) {
-        const uint32_t ew = vb1 < 2 ? e2.x : e2.y;
-        const float ve = h2f((uint16_t)(ew >> (16 * (vb1 & 1))));
+        const float ks = kscore_underflows(c, M2, Ds, es) ? 0.f : (c * sqrt_dn(fmaxf(q2, 0.f))) * vnorm;
+        return (isfinite(ks) ? ks : 0.f) * a.sens;
+      };
+      auto vscore = [&](float E, int vb) {
+        const uint32_t ew = vb < 2 ? e2.x : e2.y;
+        const float ve = h2f((uint16_t)(ew >> (16 * (vb & 1))));
         const float verr_s = sens1 ? ve : (float)((double)ve * a.sens_d);
-        sV[j] = ((c * E) * verr_s) * a.sens;
-        ++cntV;
+        return ((c * E) * verr_s) * a.sens;
+      };
+      if constexpr (K1) {
+        int nks = 0, nvs = 0, cg1 = -1, vb1 = -1;
+#pragma unroll
+        for (int cg = NCG - 1; cg >= 0; --cg)
+          if (slot_ok(A, ksl[cg])) { ++nks; cg1 = cg; }
+#pragma unroll
+        for (int vb = kVtb - 1; vb >= 0; --vb)
+          if (slot_ok(A, vsl[vb])) { ++nvs; vb1 = vb; }
+        ovf |= hm && (nks > 1 || nvs > 1);
+        subK[j] = cg1;
+        subV[j] = vb1;
+        if (ok && nks > 0) {
+          sK[0][j] = kscore(rec[1], rec[2], rec[3], rec[4], rec[5], __builtin_amdgcn_sqrtf(vsq));
+          ++cntK;
+        }
+        if (ok && vb1 >= 0 && vb1 * kVtb < nv) {
+          sV[0][j] = vscore(rec[6], vb1);
+          ++cntV;
+        }
+      } else {
+        constexpr int FMAX = 2 + 4 * NCG + kVtb;
+        const float vnorm = __builtin_amdgcn_sqrtf(vsq);
+        float es = 0.f;  // e of the page's token t*
+#pragma unroll
+        for (int f = 1; f < FMAX; ++f)
+          if (f == 1 + 4 * k_cap) es = rec[f];
+        int rk = 0, rv = 0;
+#pragma unroll
+        for (int cg = 0; cg < NCG; ++cg) {
+          if (!ok || !slot_ok(A, ksl[cg])) continue;
+          if (rk >= k_cap) { ovf = true; continue; }
+          float m[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int r = 0; r < NCG; ++r)
+            if (r == rk) {
+#pragma unroll
+              for (int f = 0; f < 4; ++f) m[f] = rec[1 + 4 * r + f];
+            }
+          const float ks = kscore(m[0], m[1], m[2], m[3], es, vnorm);
+#pragma unroll
+          for (int r = 0; r < KC; ++r)
+            if (r == rk) sK[r][j] = ks;
+          subK[j] |= cg << (4 * rk);
+          ++cntK;
+          ++rk;
+        }
+#pragma unroll
+        for (int vb = 0; vb < kVtb; ++vb) {
+          if (!ok || !slot_ok(A, vsl[vb])) continue;
+          if (rv >= v_cap) { ovf = true; continue; }
+          if (vb * kVtb < nv) {
+            float E = 0.f;
+#pragma unroll
+            for (int f = 1; f < FMAX; ++f)
+              if (f == 2 + 4 * k_cap + rv) E = rec[f];
+            const float vs = vscore(E, vb);
+#pragma unroll
+            for (int r = 0; r < VC; ++r)
+              if (r == rv) sV[r][j] = vs;
+            ++cntV;
+          }
+          subV[j] |= vb << (4 * rv);
+          ++rv;
+        }
       }
     }
   }
@@ -843,7 +903,13 @@ __global__ __launch_bounds__(256) void decode_select_wave_kernel(carekv_arena A,
   if (__any(ovf) && lane == 0) *a.err_flag = 1;
   float pk[NJ], pvv[NJ];
 #pragma unroll
-  for (int j = 0; j < NJ; ++j) { pk[j] = sK[j] >= 0.f ? sK[j] : 0.f; pvv[j] = sV[j] >= 0.f ? sV[j] : 0.f; }
+  for (int j = 0; j < NJ; ++j) {
+    pk[j] = pvv[j] = 0.f;
+#pragma unroll
+    for (int r = 0; r < KC; ++r) pk[j] = r == 0 ? (sK[0][j] >= 0.f ? sK[0][j] : 0.f) : pk[j] + (sK[r][j] >= 0.f ? sK[r][j] : 0.f);
+#pragma unroll
+    for (int r = 0; r < VC; ++r) pvv[j] = r == 0 ? (sV[0][j] >= 0.f ? sV[0][j] : 0.f) : pvv[j] + (sV[r][j] >= 0.f ? sV[r][j] : 0.f);
+  }
   const float tK = ordered_sum(pk, njp), tV = ordered_sum(pvv, njp);
   const int n_k = wave_sum_i(cntK), n_v = wave_sum_i(cntV);
 
@@ -867,21 +933,25 @@ __global__ __launch_bounds__(256) void decode_select_wave_kernel(carekv_arena A,
   const bool joint = a.policy == 1 && a.kind == 0 && haveK && haveV;
   const float divK = n_k > 0 ? fmaxf(tK / (float)n_k, kEps) : kEps;
   const float divV = n_v > 0 ? fmaxf(tV / (float)n_v, kEps) : kEps;
-  int kK[NJ], kV[NJ];
+  int kK[KC][NJ], kV[VC][NJ];
+  auto key_of = [&](float x, float div, float lam) {
+    if (!(x >= 0.f)) return -1;
+    if (do_norm) x = (x / div) * lam;
+    return (int)(__float_as_uint(x) & 0x7fffffffu);
+  };
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
-    float x = sK[j];
-    kK[j] = -1;
-    if (x >= 0.f) {
-      if (do_norm) x = (x / divK) * a.lam_k;
-      kK[j] = (int)(__float_as_uint(x) & 0x7fffffffu);
-    }
-    x = sV[j];
-    kV[j] = -1;
-    if (x >= 0.f) {
-      if (do_norm) x = (x / divV) * a.lam_v;
-      kV[j] = (int)(__float_as_uint(x) & 0x7fffffffu);
-    }
+#pragma unroll
+    for (int r = 0; r < KC; ++r) kK[r][j] = -1;
+#pragma unroll
+    for (int r = 0; r < VC; ++r) kV[r][j] = -1;
+    if (j >= njp) continue;
+#pragma unroll
+    for (int r = 0; r < KC; ++r)
+      if (K1 || r < k_cap) kK[r][j] = key_of(sK[r][j], divK, a.lam_k);
+#pragma unroll
+    for (int r = 0; r < VC; ++r)
+      if (K1 || r < v_cap) kV[r][j] = key_of(sV[r][j], divV, a.lam_v);
   }
 
   // ---- thresholds: the k-th largest key of the K keys, the V keys or both
@@ -891,22 +961,49 @@ __global__ __launch_bounds__(256) void decode_select_wave_kernel(carekv_arena A,
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
       if (j >= njp) break;
-      if (useK) n += __builtin_popcountll(__ballot(kK[j] >= t));
-      if (useV) n += __builtin_popcountll(__ballot(kV[j] >= t));
+      if (useK)
+#pragma unroll
+        for (int r = 0; r < KC; ++r)
+          if (K1 || r < k_cap) n += __builtin_popcountll(__ballot(kK[r][j] >= t));
+      if (useV)
+#pragma unroll
+        for (int r = 0; r < VC; ++r)
+          if (K1 || r < v_cap) n += __builtin_popcountll(__ballot(kV[r][j] >= t));
     }
     return n;
   };
   auto select = [&](int k, bool useK, bool useV) {
     Sel r{0u, INT_MAX, 0, true};
     if (count_ge(0, useK, useV) <= k) return r;
+    int top = 0;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      if (j >= njp) break;
+      if (useK)
+#pragma unroll
+        for (int u = 0; u < KC; ++u) top = max(top, kK[u][j]);
+      if (useV)
+#pragma unroll
+        for (int u = 0; u < VC; ++u) top = max(top, kV[u][j]);
+    }
+    top = row4_max_i(max(top, row_ror_i<2>(top)));
+    top = pair32_max_i(pair16_max_i(max(top, row_ror_i<1>(top))));
+    top = __builtin_amdgcn_readfirstlane(top);
     uint32_t tau = 0u;
-    for (int bit = 30; bit >= 0; --bit) {
+    for (int bit = 31 - __builtin_clz(top | 1); bit >= 0; --bit) {
       const uint32_t t = tau | (1u << bit);
-      if (count_ge((int)t, useK, useV) >= k) tau = t;
+      const int n = count_ge((int)t, useK, useV);
+      if (n < k) continue;
+      tau = t;
+      if (n == k) {  // every key at or above tau, no tie to rank
+        r.tau = tau;
+        return r;
+      }
     }
     r.tau = tau;
-    r.take = k - count_ge((int)tau + 1, useK, useV);
-    r.eq = count_ge((int)tau, useK, useV) - count_ge((int)tau + 1, useK, useV);
+    const int above = count_ge((int)tau + 1, useK, useV);
+    r.take = k - above;
+    r.eq = count_ge((int)tau, useK, useV) - above;
     return r;
   };
   const int takeK = haveK ? min(bud_k, n_k) : 0, takeV = haveV ? min(bud_v, n_v) : 0;
@@ -923,11 +1020,40 @@ __global__ __launch_bounds__(256) void decode_select_wave_kernel(carekv_arena A,
   // a joint selection's V ties after every K tie)
   const uint64_t below = (1ull << lane) - 1ull;
   int eq_runK = 0, eq_runV = 0;
-  if (joint && sk.on && sk.take < sk.eq) {
+  const bool rankK = sk.on && sk.take < sk.eq, rankV = sv.on && sv.take < sv.eq;  // ties to rank
+  if (joint && rankK) {
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
-      if (j < njp) eq_runV += __builtin_popcountll(__ballot(kK[j] >= 0 && (uint32_t)kK[j] == sk.tau));
+      if (j < njp)
+#pragma unroll
+        for (int r = 0; r < KC; ++r) eq_runV += __builtin_popcountll(__ballot(kK[r][j] >= 0 && (uint32_t)kK[r][j] == sk.tau));
   }
+  // the candidates of one kind that a lane's page j takes (bit r: rank r)
+  auto taken = [&](const auto& key, int j, const Sel& sel, bool rank, int& eq_run) {
+    constexpr int N = sizeof(key) / sizeof(key[0]);
+    unsigned bits = 0;
+    int before = eq_run;
+    if (rank) {
+#pragma unroll
+      for (int r = 0; r < N; ++r) {
+        const uint64_t e = __ballot(key[r][j] >= 0 && (uint32_t)key[r][j] == sel.tau);
+        before += __builtin_popcountll(e & below);
+        eq_run += __builtin_popcountll(e);
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < N; ++r) {
+      if (!sel.on || key[r][j] < 0) continue;
+      const uint32_t x = (uint32_t)key[r][j];
+      bool t = x > sel.tau;
+      if (x == sel.tau) {
+        t = !rank || before < sel.take;
+        ++before;
+      }
+      if (t) bits |= 1u << r;
+    }
+    return bits;
+  };
   uint8_t* maskq = a.mask + bq * a.Pmax;
   unsigned selK[NJ], selV[NJ];
 #pragma unroll
@@ -935,24 +1061,14 @@ __global__ __launch_bounds__(256) void decode_select_wave_kernel(carekv_arena A,
     selK[j] = selV[j] = 0u;
     if (j >= njp) continue;
     const int p = lane + 64 * j;
-    const bool eqk = sk.on && kK[j] >= 0 && (uint32_t)kK[j] == sk.tau;
-    const bool eqv = sv.on && kV[j] >= 0 && (uint32_t)kV[j] == sv.tau;
-    const uint64_t bk_eq = __ballot(eqk), bv_eq = __ballot(eqv);
-    const int rk = eq_runK + __builtin_popcountll(bk_eq & below);
-    const int rv = eq_runV + __builtin_popcountll(bv_eq & below);
-    eq_runK += __builtin_popcountll(bk_eq);
-    eq_runV += __builtin_popcountll(bv_eq);
-    bool tk = false, tv = false;
-    if (sk.on && kK[j] >= 0) tk = (uint32_t)kK[j] > sk.tau || (eqk && rk < sk.take);
-    if (sv.on && kV[j] >= 0) tv = (uint32_t)kV[j] > sv.tau || (eqv && rv < sv.take);
-    selK[j] = tk ? 1u : 0u;
-    selV[j] = tv ? 1u : 0u;
+    selK[j] = taken(kK, j, sk, rankK, eq_runK);
+    selV[j] = taken(kV, j, sv, rankV, eq_runV);
     if (p < np) maskq[p] = (uint8_t)(selK[j] | (selV[j] << 4));
   }
   if (a.read_counts) {
     int ck = 0, cvb = 0;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) { ck += (int)selK[j]; cvb += (int)selV[j]; }
+    for (int j = 0; j < NJ; ++j) { ck += __popc(selK[j]); cvb += __popc(selV[j]); }
     ck = wave_sum_i(ck);
     cvb = wave_sum_i(cvb);
     if (lane == 0 && L > 0.f) {
@@ -969,11 +1085,21 @@ __global__ __launch_bounds__(256) void decode_select_wave_kernel(carekv_arena A,
     for (int j = 0; j < NJ; ++j) {
       if (j >= njp) break;
       const int p = lane + 64 * j;
-      const bool on = kind == 0 ? selK[j] != 0u : selV[j] != 0u;
-      const uint64_t bal = __ballot(on);
-      const int pos = run + __builtin_popcountll(bal & below);
-      run += __builtin_popcountll(bal);
-      if (on && pos < a.diag_cap) diagp[pos] = (kind << 30) | (p << 3) | (kind == 0 ? cgK[j] : vbV[j]);
+      const unsigned bits = kind == 0 ? selK[j] : selV[j];
+      const int sub = kind == 0 ? subK[j] : subV[j];
+      int pos = run;
+#pragma unroll
+      for (int r = 0; r < kVtb; ++r) {
+        const uint64_t bal = __ballot(bits >> r & 1u);
+        pos += __builtin_popcountll(bal & below);
+        run += __builtin_popcountll(bal);
+      }
+#pragma unroll
+      for (int r = 0; r < kVtb; ++r)
+        if (bits >> r & 1u) {
+          if (pos < a.diag_cap) diagp[pos] = (kind << 30) | (p << 3) | (sub >> (4 * r) & 15);
+          ++pos;
+        }
     }
   }
   for (int i = run + lane; i < a.diag_cap; i += 64) diagp[i] = -1;
@@ -985,19 +1111,25 @@ int launch_decode_select(const carekv_arena& A, const DecodeArgs& a, hipStream_t
   const size_t lds = (a.correction && a.ncand <= kLdsCand) ? (size_t)a.ncand * sizeof(float) : 0;
   const bool px = a.correction && a.proxy;
   const bool k1 = a.k_cap == 1 && a.v_cap == 1;
-  // rows of at most 256 pages with one K and one V slot, and enough query
-  // columns to fill the GPU with waves (or short rows, where the work-group
-  // form's fixed cost dominates): a wave per query.  CAREKV_SELECT_WAVE=0
-  // keeps the work-group form, =2 takes the wave form for every row it covers.
+  // rows of at most 256 pages, and enough query columns to fill the GPU with
+  // waves (or short rows, where the work-group form's fixed cost dominates):
+  // a wave per query.  CAREKV_SELECT_WAVE=0 keeps the work-group form, =2
+  // takes the wave form for every row it covers.
   const char* env = getenv("CAREKV_SELECT_WAVE");
   const int wmode = env ? env[0] - '0' : 1;
   const long cols = (long)pairs * a.GQ;
-  if (wmode != 0 && a.correction && !px && k1 && (a.policy == 0 || a.policy == 1) && !a.adaptive_score &&
-      a.Pmax <= 256 && a.nsplit <= 256 && a.F == 7 && (wmode == 2 || cols >= 2048 || a.Pmax <= 64)) {
+  if (wmode != 0 && a.correction && !px && (a.policy == 0 || a.policy == 1) && !a.adaptive_score && a.Pmax <= 256 &&
+      a.nsplit <= 256 && a.F == 2 + 4 * a.k_cap + a.v_cap && a.k_cap <= A.head_dim / 32 && a.v_cap <= kVtb &&
+      (wmode == 2 || cols >= 2048 || a.Pmax <= 64)) {
     const int ngq = (a.GQ + 3) / 4;
     const dim3 gw(((pairs + kXcd - 1) / kXcd) * kXcd * ngq);
-    if (A.head_dim == 64) hipLaunchKernelGGL((decode_select_wave_kernel<64>), gw, dim3(kBlock), 0, s, A, a);
-    else if (A.head_dim == 128) hipLaunchKernelGGL((decode_select_wave_kernel<128>), gw, dim3(kBlock), 0, s, A, a);
+    auto wave = [&](auto d) {
+      constexpr int D = decltype(d)::value;
+      if (k1) hipLaunchKernelGGL((decode_select_wave_kernel<D, true>), gw, dim3(kBlock), 0, s, A, a);
+      else hipLaunchKernelGGL((decode_select_wave_kernel<D, false>), gw, dim3(kBlock), 0, s, A, a);
+    };
+    if (A.head_dim == 64) wave(std::integral_constant<int, 64>{});
+    else if (A.head_dim == 128) wave(std::integral_constant<int, 128>{});
     else {
       set_error("unsupported head_dim %d", A.head_dim);
       return CAREKV_EINVAL;
