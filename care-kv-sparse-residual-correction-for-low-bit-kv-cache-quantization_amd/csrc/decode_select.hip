@@ -217,7 +217,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
   constexpr int FMAX = 2 + 4 * NCG + kVtb;
   __shared__ BlockScratch bs;
   __shared__ int hist[2][256];  // one histogram per wave pair
-  __shared__ float s_qs[NCG * 64];  // q_cg P per channel group (sketch proxy)
+  __shared__ __align__(16) float s_qs[NCG * 68];  // q_cg P per channel group (sketch proxy; padded: lanes read different groups)
   extern __shared__ float s_cand[];  // ncand floats when they fit (size set at launch)
   const int GQ = a.GQ;
   // prefill rows: the latest (longest) rows first (a window keeps its XCD)
@@ -288,7 +288,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
       float acc = 0.f;
       if (qg)
         for (int c = 0; c < 32; ++c) acc = fmaf(h2f(qg[cg * 32 + c]), a.sketch_proj[c * skd + j], acc);
-      s_qs[cg * 64 + j] = acc;
+      s_qs[cg * 68 + j] = acc;
     }
     __syncthreads();
   }
@@ -316,19 +316,40 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
       const bool ok = L > 0.f && A.valid[pg] > 0 && A.has_meta[pg];
       float4 px = make_float4(0.f, 0.f, 0.f, 0.f);  // mass, boundary, vdiff
       if (ok) px = *reinterpret_cast<const float4*>(a.prox + (bq * a.Pmax + p) * 4);
-      int rk = 0;
-#pragma unroll 1
+      // the page's stored channel groups in rank order, 4 bits each: a lane
+      // walks its own slots (over the channel groups, with one slot a page,
+      // three of four passes were idle), a sketch row 16 bytes at a time
+      int ksl[NCG], cgs = 0, rk = 0;
+      load_slots<NCG>(ksl, A.k_slot + pg * NCG);
+#pragma unroll
       for (int cg = 0; cg < NCG; ++cg) {
-        if (!ok || !slot_ok(A, A.k_slot[pg * NCG + cg])) continue;
+        if (!ok || !slot_ok(A, ksl[cg])) continue;
         if (rk >= k_cap) { ovf = true; continue; }
+        cgs |= cg << (4 * rk);
+        ++rk;
+      }
+      const int nk = rk;
+#pragma unroll 1
+      for (rk = 0; rk < nk; ++rk) {
+        const int cg = cgs >> (4 * rk) & 15;
         const uint16_t* ks = A.k_sketch + (pg * NCG + cg) * skd;
+        const float* qs = s_qs + cg * 68;
         float dot = 0.f;
-        for (int j = 0; j < skd; ++j) dot = fmaf(s_qs[cg * 64 + j], h2f(ks[j]), dot);
+        if ((skd & 7) == 0) {
+#pragma unroll 4
+          for (int j = 0; j < skd; j += 8) {
+            const uint4 v = *reinterpret_cast<const uint4*>(ks + j);
+            const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) dot = fmaf(qs[j + e], h2f((uint16_t)(u[e >> 1] >> (16 * (e & 1)))), dot);
+          }
+        } else {
+          for (int j = 0; j < skd; ++j) dot = fmaf(qs[j], h2f(ks[j]), dot);
+        }
         const float kp = (((px.x * fabsf(dot)) * px.y) * px.z) * a.sens;
         sc[p * k_cap + rk] = kp;
         sumK += kp;
         ++cntK;
-        ++rk;
       }
       for (; rk < k_cap; ++rk) sc[p * k_cap + rk] = -1.f;
     }
@@ -412,7 +433,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
     float r[FMAX];
     const float* rp = recq + (long)p * F;
 #pragma unroll
-    for (int f = 0; f < FMAX; ++f) r[f] = f < F ? rp[f] : 0.f;
+    for (int f = 0; f < FMAX; ++f) r[f] = f < F && (!PX || f == 0 || f >= 2 + 4 * k_cap) ? rp[f] : 0.f;
     const bool ok = L > 0.f && nv > 0 && hm;
     const float c = exp2_dn(ok ? r[0] - M : -INFINITY) * invL;
     const float vnorm = __builtin_amdgcn_sqrtf(vsq);
