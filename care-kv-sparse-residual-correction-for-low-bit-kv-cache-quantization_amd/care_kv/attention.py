@@ -141,16 +141,20 @@ def decode_read_mode(cfg: CacheConfig, layer: int):
     return any_read_budget(cfg), knobs
 
 
-def default_split_pages(max_pages: int, rows: int) -> int:
-    """Pages per work-group of the streaming pass, a multiple of 16 (4 waves
-    x 4-page windows): long enough that each wave's start-up (q staging, the
-    first window's loads, the split merge) spreads over several windows --
-    half a row, at most 256 pages -- and short enough that the grid keeps at
-    least CAREKV_DECODE_MIN_WGS (default 1024: four per CU) work-groups."""
+def default_split_pages(max_pages: int, rows: int, step: int = 16) -> int:
+    """Pages per work-group of the streaming pass, a multiple of ``step``
+    (16: 4 waves x 4-page windows of the 4-query-head kernel; 4 where the
+    kernel takes a page per wave): long enough that each wave's start-up (q
+    staging, the first window's loads, the split merge) spreads over several
+    windows -- half a row, at most 256 pages -- and short enough that the grid
+    keeps at least CAREKV_DECODE_MIN_WGS (default 1024: four per CU)
+    work-groups."""
     min_wgs = max(1, int(os.environ.get("CAREKV_DECODE_MIN_WGS", "1024")))
     P, R = max(1, max_pages), max(1, rows)
-    sp = max(16, min(256, -(-P // 2), (P * R) // min_wgs))
-    return (sp + 15) // 16 * 16
+    sp = max(step, min(256, -(-P // 2), (P * R) // min_wgs))
+    if sp < 16:  # shorter splits pay for their partials only where they spread over idle CUs
+        sp = max(step, min(16, 2 * P * R // min_wgs))
+    return (sp + step - 1) // step * step
 
 
 def _read_params(cache: CAREKVCache, layer: int, knobs: ReadKnobs, *, batch: int, n_heads: int, correction: bool,
@@ -279,7 +283,13 @@ def decode_attention(cache: CAREKVCache, layer: int, q: torch.Tensor, seqs: Opti
             cache._row_tables.clear()
         cache._row_tables[key] = meta
     if split_pages is None:
-        split_pages = default_split_pages(max_np, B * cfg.num_kv_heads)
+        # more than 4 query heads per kv head, or fp16 pages: the kernel takes a
+        # page per wave, so rows too few to fill the GPU split down to 4 pages
+        # (4 rows of 32 pages: 27.9 us a step against 38.1 with 16-page splits;
+        # 128 rows of 144 pages: 66.0 us with 20 against 73 with 32; 32 rows of
+        # 250 pages keep 16: 58 us against 60 with 8)
+        page_wave = cfg.num_heads > 4 * cfg.num_kv_heads or (cache.hat and not cache.kivi_packed)
+        split_pages = default_split_pages(max_np, B * cfg.num_kv_heads, step=4 if page_wave else 16)
     dp = _read_params(cache, layer, knobs, batch=B, n_heads=Hq, correction=correction, split_pages=split_pages,
                       max_pages=max_np, seq_ptr=meta[0].data_ptr(), np_ptr=meta[1].data_ptr())
     if cache.kivi_packed and B:  # the packed prefix and the fp16 tail run as separate page ranges

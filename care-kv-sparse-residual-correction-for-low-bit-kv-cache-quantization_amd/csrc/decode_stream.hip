@@ -111,26 +111,30 @@ void decode_stream_kernel(carekv_arena A, DecodeArgs a) {
   for (; p < p_end; p += 4) {
     const PageRegs<D, BITS> cur = nx;
     const PageMeta<NCG> cm = meta_from_lanes<NCG>(nmv, A);
-    if (p + 4 < p_end) {
-      load_page_regs<D, BITS, SM>(nx, rr, p + 4, ln, lj);
-      nmv = meta_lanes_load<NCG>(A, pg_base + p + 4, lane);
-    }
     const float ckm = h2f((uint16_t)cm.kmaster), cvm = h2f((uint16_t)cm.vmaster);
     const int nv = PF ? min(cm.nv, er.ntok - p * kPage) : cm.nv;
-    if (nv <= 0) continue;
-    // K residual rows of the stored slots, issued before the page math
-    uint32_t krow[NCG];
-    if (corr && cm.meta && !a.proxy) {
+    // K residual rows and scales of the stored slots, issued before the next
+    // page's loads: loads return in order, so behind them the records would
+    // wait for the next page too, and a scale loaded where it is used would
+    // cost each slot a round trip of its own
+    uint32_t krow[NCG], ksc[NCG];
+    if (nv > 0 && corr && cm.meta && !a.proxy) {
 #pragma unroll
       for (int cg = 0; cg < NCG; ++cg) {
-        krow[cg] = 0u;
+        krow[cg] = ksc[cg] = 0u;
         if (cm.ksl[cg] >= 0) {
           const long so = (long)seq * A.n_slots + cm.ksl[cg];
           const __amdgpu_buffer_rsrc_t r = make_rsrc(A.k_res + so * G::KSB, G::KSB);
           krow[cg] = __builtin_amdgcn_raw_buffer_load_b32(r, ln * 16 + lj * 4, 0, 0);
+          ksc[cg] = A.k_res_scale[so];
         }
       }
     }
+    if (p + 4 < p_end) {
+      load_page_regs<D, BITS, SM>(nx, rr, p + 4, ln, lj);
+      nmv = meta_lanes_load<NCG>(A, pg_base + p + 4, lane);
+    }
+    if (nv <= 0) continue;
     // ---- S = K_hat q
     const _Float16 ks = lane_scale<SM>(cur.ksc, ckm), vs = lane_scale<SM>(cur.vsc, cvm);
     const float4_t sacc = page_scores<D, BITS>(cur.kw, ks, qB);
@@ -215,7 +219,6 @@ void decode_stream_kernel(carekv_arena A, DecodeArgs a) {
         if (slot < 0) continue;
         if (rk >= a.k_cap) break;  // flagged by the select kernel
         if (a.proxy) { ++rk; continue; }  // the sketch proxy scores K slots without the moments
-        const long so = (long)seq * A.n_slots + slot;
         const float4_t racc = kslot_dot_w(krow[cg], sqr, D, cg, ln, lj);
         // moments of u = racc * e over the tokens other than t* (dS = racc
         // * f scales them by f^2): M2 = sum u^2, M3 = sum u^2 e, M4 = sum
@@ -237,7 +240,7 @@ void decode_stream_kernel(carekv_arena A, DecodeArgs a) {
         // M2, M3, M4, D*
         const float mj = moments_reduce4(M2, M3, M4, Ds);
         if (ln < GQ) {
-          const float f = h2f(A.k_res_scale[so]) * a.inv_sqrt_d;
+          const float f = h2f((uint16_t)ksc[cg]) * a.inv_sqrt_d;
           rec[1 + 4 * rk + lj] = mj * (f * f);
         }
         ++rk;
