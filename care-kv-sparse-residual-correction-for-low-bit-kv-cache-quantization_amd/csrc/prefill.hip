@@ -51,6 +51,8 @@ __global__ __launch_bounds__(256, 3) void prefill_attn_kernel(PrefillArgs a) {
   constexpr int KBUF = KT * KRS, VBUF = KT * VRS, BUF = KBUF + VBUF;
   constexpr int CHR = D / 8;          // 16-byte chunks per row
   constexpr int NCH = 2 * KT * CHR / 256;  // chunks a thread stages per tile
+  constexpr float kSlack = 256.f;     // weights up to 2^8, far inside fp16
+  constexpr float kLow = -1e30f;      // below any score; finite, so that a masked score's weight is 0 from the first tile
   __shared__ __align__(16) char lds[2 * BUF];
   typedef short short4_t __attribute__((ext_vector_type(4)));
   typedef __attribute__((address_space(3))) short4_t lds_short4;
@@ -109,7 +111,7 @@ __global__ __launch_bounds__(256, 3) void prefill_attn_kernel(PrefillArgs a) {
     }
   };
 
-  float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.f, 0.f};
+  float m_run[2] = {kLow, kLow}, l_run[2] = {0.f, 0.f};
   float4_t o[2][DT];
 #pragma unroll
   for (int qb = 0; qb < 2; ++qb)
@@ -167,32 +169,43 @@ __global__ __launch_bounds__(256, 3) void prefill_attn_kernel(PrefillArgs a) {
               if (o >= lim_t || o > lim_q) s[tt][qb][i] = -INFINITY;
             }
         }
-        // a chain of three-operand maxima over the lane's 16 scores
-        float mx = s[0][qb][0];
+      }
+      float ls[2];
+      auto weigh = [&]() {  // the weights and this lane's sums of them (its tokens; over the lane groups at the end)
 #pragma unroll
-        for (int k = 1; k < 4 * TT; k += 2) {
-          const int k2 = k + 1 < 4 * TT ? k + 1 : k;
-          mx = fmaxf(fmaxf(mx, s[k / 4][qb][k % 4]), s[k2 / 4][qb][k2 % 4]);
+        for (int qb = 0; qb < 2; ++qb) {
+          ls[qb] = 0.f;
+#pragma unroll
+          for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              p[tt][qb][i] = __builtin_amdgcn_exp2f(fmaf(s[tt][qb][i], c, -m_run[qb]));
+              ls[qb] += p[tt][qb][i];
+            }
         }
-        mx = pair32_max(pair16_max(mx)) * c;
-        const float m_new = fmaxf(m_run[qb], mx);  // finite: token 0 is visible to every query
-        const float f = __builtin_amdgcn_exp2f(m_run[qb] - m_new);
-        m_run[qb] = m_new;
-        float ls = 0.f;
+      };
+      weigh();
+      // The reference maximum moves only when the weights outgrow it (a lane's
+      // sum over kSlack, so no weight passes it): most tiles need no maximum,
+      // no reduction over the lane groups and no rescale.  The first tile
+      // always comes here (m_run = kLow makes its sums infinite).
+      if (__builtin_expect(__any(ls[0] > kSlack || ls[1] > kSlack), 0)) {
 #pragma unroll
-        for (int tt = 0; tt < TT; ++tt)
+        for (int qb = 0; qb < 2; ++qb) {
+          float mx = s[0][qb][0];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float e = __builtin_amdgcn_exp2f(fmaf(s[tt][qb][i], c, -m_new));
-            p[tt][qb][i] = e;
-            ls += e;
-          }
-        l_run[qb] = l_run[qb] * f + ls;  // this lane's tokens; summed over the lane groups at the end
-        if (__builtin_expect(__any(f != 1.f), 0)) {
+          for (int k = 1; k < 4 * TT; ++k) mx = fmaxf(mx, s[k / 4][qb][k % 4]);
+          const float m_new = fmaxf(m_run[qb], pair32_max(pair16_max(mx)) * c);
+          const float f = __builtin_amdgcn_exp2f(m_run[qb] - m_new);
+          m_run[qb] = m_new;
+          l_run[qb] *= f;
 #pragma unroll
           for (int dt = 0; dt < DT; ++dt) o[qb][dt] *= f;
         }
+        weigh();
       }
+      l_run[0] += ls[0];
+      l_run[1] += ls[1];
       __builtin_amdgcn_s_setprio(1);
       // ---- O^T += V_hat^T P^T, 32 tokens per step
 #pragma unroll
