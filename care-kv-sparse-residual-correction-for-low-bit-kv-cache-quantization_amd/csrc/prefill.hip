@@ -8,13 +8,23 @@
 // (latest) query blocks of every (sequence, head) first.  K and V tiles of 32
 // tokens are staged in LDS (double buffered, one barrier per tile; the next
 // tile's global loads are in flight while the current one is used); at
-// D = 128, 160 VGPRs and 35 KB of LDS, three work-groups share a CU:
+// D = 128, 168 VGPRs and 35 KB of LDS, three work-groups share a CU:
 //   * S^T = K_hat Q^T: A = K tile rows (one 16-byte LDS read per lane and
 //     32-dim step), B = Q^T held in registers; lane l receives the scores of
 //     tokens 16tt + 4(l/16) + i for query l % 16 of a 16-query sub-block;
 //   * the online softmax runs per query column in fp32 on base-2 logits
 //     (scores scaled by log2(e)/sqrt(D) after the fp32 product, as the
 //     reference divides the fp32 product by sqrt(D));
+//     The weights are exp2(x - m) with a reference maximum m that moves only
+//     when a tile's weights outgrow it by 2^8: the maximum, its reduction over
+//     the lane groups, the rescale factor and its test were a third of the
+//     loop's VALU work (of about 120 instructions a tile 66 are left),
+//     which bounds the kernel with its 16 exponentials a tile.  B = 4, 40
+//     heads, T = 8192, D = 128: 3613 -> 3279 us; B = 8, 32 / 4 heads, T = 2047,
+//     D = 64: 226 -> 189 us.  The fp16 weights keep 11 bits each, but the
+//     largest is no longer exactly 1, as in the reference, whose normalised
+//     weights are rounded wherever they fall: 2.7e-4 against 2.5e-4 from a
+//     64-bit evaluation, most of both the output's own rounding;
 //   * O^T += V_hat^T P^T: the weights are already in the B layout (the 8 k
 //     values of a lane are tokens 4(l/16) + i of two 16-token tiles), and
 //     the A operand V_hat^T comes from the token-major V tile through the
