@@ -119,6 +119,14 @@ def load(path: str | None = None):
                                              vp, vp]
         lib.carekv_append_rows.restype = C.c_int
         lib.carekv_append_rows.argtypes = [C.POINTER(Arena), vp, vp, vp, i32, vp]
+        lib.carekv_append_rows_open.restype = C.c_int
+        lib.carekv_append_rows_open.argtypes = [C.POINTER(Arena), vp, vp, vp, i32, vp, vp, vp]
+        lib.carekv_open_rows.restype = C.c_int
+        lib.carekv_open_rows.argtypes = [C.POINTER(Arena), vp, vp, vp, i32, i32, i32, vp, vp, vp]
+        lib.carekv_reset_sequence.restype = C.c_int
+        lib.carekv_reset_sequence.argtypes = [vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, vp]
+        lib.carekv_rope_heads.restype = C.c_int
+        lib.carekv_rope_heads.argtypes = [vp, vp, vp, vp, vp, i64, i64, i32, i32, i32, i32, i32, vp, vp, vp, vp]
         lib.carekv_decode_workspace_bytes.restype = i64
         lib.carekv_decode_workspace_bytes.argtypes = [C.POINTER(Arena), C.POINTER(DecodeParams)]
         lib.carekv_decode_attn.restype = C.c_int

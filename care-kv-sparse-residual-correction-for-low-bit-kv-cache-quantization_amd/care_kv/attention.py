@@ -151,6 +151,8 @@ def default_split_pages(max_pages: int, rows: int, step: int = 16) -> int:
     work-groups."""
     min_wgs = max(1, int(os.environ.get("CAREKV_DECODE_MIN_WGS", "1024")))
     P, R = max(1, max_pages), max(1, rows)
+    if P * R > 32 * min_wgs:  # the grid is full either way, and fewer partials keep the workspace small
+        step = max(step, 16)
     sp = max(step, min(256, -(-P // 2), (P * R) // min_wgs))
     if sp < 16:  # shorter splits pay for their partials only where they spread over idle CUs
         sp = max(step, min(16, 2 * P * R // min_wgs))
@@ -282,6 +284,7 @@ def decode_attention(cache: CAREKVCache, layer: int, q: torch.Tensor, seqs: Opti
         if len(cache._row_tables) > 64:
             cache._row_tables.clear()
         cache._row_tables[key] = meta
+    short = False
     if split_pages is None:
         # more than 4 query heads per kv head, or fp16 pages: the kernel takes a
         # page per wave, so rows too few to fill the GPU split down to 4 pages
@@ -290,6 +293,7 @@ def decode_attention(cache: CAREKVCache, layer: int, q: torch.Tensor, seqs: Opti
         # 250 pages keep 16: 58 us against 60 with 8)
         page_wave = cfg.num_heads > 4 * cfg.num_kv_heads or (cache.hat and not cache.kivi_packed)
         split_pages = default_split_pages(max_np, B * cfg.num_kv_heads, step=4 if page_wave else 16)
+        short = page_wave
     dp = _read_params(cache, layer, knobs, batch=B, n_heads=Hq, correction=correction, split_pages=split_pages,
                       max_pages=max_np, seq_ptr=meta[0].data_ptr(), np_ptr=meta[1].data_ptr())
     if cache.kivi_packed and B:  # the packed prefix and the fp16 tail run as separate page ranges
@@ -309,6 +313,8 @@ def decode_attention(cache: CAREKVCache, layer: int, q: torch.Tensor, seqs: Opti
         dp.phase_events = ctypes.cast(ev_arr, ctypes.c_void_p)
     lib = _lib.load()
     a = cache.arena(layer)
+    if no_alloc and short and int(lib.carekv_decode_workspace_bytes(a, dp)) > _lib.STATIC_SCRATCH_BYTES:
+        dp.split_pages = default_split_pages(max_np, B * cfg.num_kv_heads)  # fewer partials
     if out is None:
         out = torch.empty(B, Hq, D, dtype=torch.float16, device=dev)
     diag = torch.empty(B, Hq, diag_cap, dtype=torch.int32, device=dev) if diag_cap > 0 else None

@@ -20,6 +20,7 @@ deterministically), so appends and decode never read device memory back.
 from __future__ import annotations
 
 import math
+import operator
 from dataclasses import dataclass, field
 from typing import Dict, List, Optional, Sequence, Tuple
 
@@ -354,11 +355,12 @@ class CAREKVCache:
 
     def reset_sequence(self, seq: int):
         """Forget a sequence slot (pages, metadata, residual slots)."""
-        self.valid[:, :, seq].zero_()
-        self.has_meta[:, :, seq].zero_()
-        self.k_slot[:, :, seq].fill_(-1)
-        self.v_slot[:, :, seq].fill_(-1)
-        self.next_slot[seq].zero_()
+        seq = range(self.n_seq)[operator.index(seq)]  # (a negative slot counts from the end)
+        lib = _lib.load()
+        _lib.check(lib.carekv_reset_sequence(
+            self.valid.data_ptr(), self.has_meta.data_ptr(), self.k_slot.data_ptr(), self.v_slot.data_ptr(),
+            self.next_slot.data_ptr(), self.cfg.num_layers * self.cfg.num_kv_heads, self.n_seq, self.cfg.max_pages,
+            self.ncg, self.nvb, seq, _lib.stream_ptr(self.device)), "carekv_reset_sequence")
         self._freed.pop((seq, 0), None)
         self._freed.pop((seq, 1), None)
         self.next_page[:, :, seq] = 0
@@ -469,28 +471,12 @@ class CAREKVCache:
             _lib.check_status(ws, 4 * n_jobs, "carekv_store_prefill")
         else:
             self.status.watch(ws, 4 * n_jobs, "carekv_store_prefill")
-        if self.rescale_open:  # the last page stays open: keep its rows' fp16 group scales
-            last = T - (n_new - 1) * ps
-            if last < ps:
-                G = D // cfg.group_size
-                tail = torch.cat([K[:, :, (n_new - 1) * ps:], V[:, :, (n_new - 1) * ps:]], 0).to(F16).contiguous()
-                codes = torch.empty(2 * B * H * last, D, dtype=torch.int8, device=self.device)
-                sc = torch.empty(2 * B * H * last, G, dtype=F16, device=self.device)
-                _lib.check(lib.carekv_quantize_rows(tail.data_ptr(), 2 * B * H * last, D, cfg.base_bits, 32, 0,
-                                                    codes.data_ptr(), sc.data_ptr(), _lib.stream_ptr(self.device)),
-                           "carekv_quantize_rows (open page scales)")
-                sc = sc.view(2, B, H, last, G)
-                sl = torch.tensor(seqs, device=self.device)
-                self.open_ks[layer][:, sl, :last] = sc[0].transpose(0, 1)
-                self.open_vs[layer][:, sl, :last] = sc[1].transpose(0, 1)
-        if self.streaming_store:  # the last page stays open: keep its true rows
-            last = T - (n_new - 1) * ps
-            sl = torch.tensor(seqs, device=self.device)
-            self.open_k[layer, sl] = 0
-            self.open_v[layer, sl] = 0
-            if last < ps:
-                self.open_k[layer, sl, :, :last] = K[:, :, (n_new - 1) * ps:].to(F16)
-                self.open_v[layer, sl, :, :last] = V[:, :, (n_new - 1) * ps:].to(F16)
+        last = T - (n_new - 1) * ps
+        if self.streaming_store or (self.rescale_open and last < ps):
+            # the last page stays open: keep its true rows and their fp16 group scales
+            ok, ov = (self.open_k[layer].data_ptr(), self.open_v[layer].data_ptr()) if self.streaming_store else (None, None)
+            _lib.check(lib.carekv_open_rows(a, Kp.data_ptr(), Vp.data_ptr(), rows_d.data_ptr(), B, n_new, last, ok, ov,
+                                            _lib.stream_ptr(self.device)), "carekv_open_rows")
         if hats is not None:
             return hats[0] if B > 1 else hats[0][0], hats[1] if B > 1 else hats[1][0]
         return None
@@ -533,26 +519,16 @@ class CAREKVCache:
                         -1).reshape(B * H, 4).astype(np.int32)
         fb, fh = np.nonzero(offs + 1 == ps)
         filled = [(int(sarr[b_]), int(h_), int(pid[b_, h_])) for b_, h_ in zip(fb, fh)]  # the pages the appends fill
-        offs = offs.reshape(B * H).astype(np.int64)
-        # one upload: the page destinations (int32 [B*H][4]) and, with the
-        # streaming store, the rows of the open-page buffers (seq, head, offset)
-        # flattened (int64 [B*H])
-        n = B * H
-        buf = np.empty(2 * n + (n if self.streaming_store else 0), dtype=np.int64)
-        buf[:2 * n].view(np.int32)[:] = dest.reshape(-1)
-        if self.streaming_store:
-            buf[2 * n:] = (dest[:, 0].astype(np.int64) * H + dest[:, 1]) * ps + offs
-        buf_d = to_device(buf, self.device)
-        dest_d = buf_d[:2 * n].view(torch.int32)
+        dest_d = to_device(dest, self.device)
         kk = k.to(F16).contiguous().view(B * H, D)
         vv = v.to(F16).contiguous().view(B * H, D)
         lib = _lib.load()
-        _lib.check(lib.carekv_append_rows(self.arena(layer), kk.data_ptr(), vv.data_ptr(), dest_d.data_ptr(), B * H,
-                                          _lib.stream_ptr(self.device)), "carekv_append_rows")
-        if self.streaming_store:
-            rows = buf_d[2 * n:]
-            self.open_k[layer].view(-1, D).index_copy_(0, rows, kk)
-            self.open_v[layer].view(-1, D).index_copy_(0, rows, vv)
+        args = (self.arena(layer), kk.data_ptr(), vv.data_ptr(), dest_d.data_ptr(), B * H)
+        if not self.streaming_store:
+            _lib.check(lib.carekv_append_rows(*args, _lib.stream_ptr(self.device)), "carekv_append_rows")
+        else:
+            _lib.check(lib.carekv_append_rows_open(*args, self.open_k[layer].data_ptr(), self.open_v[layer].data_ptr(),
+                                                   _lib.stream_ptr(self.device)), "carekv_append_rows_open")
             if filled:
                 self._streaming_fill_store(layer, filled)
 

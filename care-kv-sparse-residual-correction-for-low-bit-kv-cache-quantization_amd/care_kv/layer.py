@@ -26,6 +26,7 @@ from typing import Any, Dict, Optional, Sequence, Tuple
 import torch
 from torch import Tensor, nn
 
+from . import _lib
 from .attention import (debug_stats_enabled, decode_attention, decode_read_mode, get_debug_stats,  # noqa: F401
                         get_imp_per_layer, importance_probe, prefill_correction, reset_debug_stats)
 from .cache import CAREKVCache
@@ -78,6 +79,14 @@ def _rope(q: Tensor, k: Tensor, cos: Tensor, sin: Tensor) -> Tuple[Tensor, Tenso
     return q * c + rot(q) * s, k * c + rot(k) * s
 
 
+def _rope_tables(cos: Tensor, sin: Tensor, B: int, T: int, D: int) -> bool:
+    """Whether carekv_rope_heads reads these tables: (B or 1, T, D) on the
+    device, rows of consecutive values at the same strides, 8-byte aligned."""
+    return (cos.dim() == 3 and cos.shape == sin.shape and cos.shape[0] in (1, B) and tuple(cos.shape[1:]) == (T, D)
+            and cos.is_cuda and sin.is_cuda and cos.stride() == sin.stride() and cos.stride(2) == 1
+            and (cos.data_ptr() | sin.data_ptr()) % 8 == 0 and cos.stride(0) % 4 == 0 and cos.stride(1) % 4 == 0)
+
+
 class CAREKVLayer(nn.Module):
     """Drop-in attention layer over the CARE-KV cache (layer.py:147-183)."""
 
@@ -102,6 +111,31 @@ class CAREKVLayer(nn.Module):
         K = (hidden @ self.W_K.T).reshape(B, T, Hkv, D).transpose(1, 2)
         V = (hidden @ self.W_V.T).reshape(B, T, Hkv, D).transpose(1, 2)
         return Q, K, V
+
+    def _heads(self, hidden: Tensor, position_embeddings) -> Tuple[Tensor, Tensor, Tensor]:
+        """hidden (B, T, model_dim) -> Q (B, Hq, T, D), K / V (B, Hkv, T, D),
+        fp16 contiguous, Q and K under RoPE when position_embeddings is given.
+        fp16 projections with (B or 1, T, D) tables go through
+        carekv_rope_heads in one launch, with the same roundings; other
+        forms take the elementwise operations."""
+        cfg = self.cfg
+        B, T, _ = hidden.shape
+        Hq, Hkv, D = cfg.num_heads, cfg.num_kv_heads, cfg.head_dim
+        Q, K, V = self._project(hidden)
+        cos, sin = (None, None) if position_embeddings is None else (x.to(Q.dtype) for x in position_embeddings)
+        q, k, v = (x.transpose(1, 2) for x in (Q, K, V))  # the projections' own layout
+        if (q.dtype == F16 and q.is_cuda and B * T > 0 and all(x.is_contiguous() for x in (q, k, v))
+                and (cos is None or _rope_tables(cos, sin, B, T, D))):
+            qo, ko, vo = (torch.empty(B, h, T, D, dtype=F16, device=q.device) for h in (Hq, Hkv, Hkv))
+            ptr = [None, None, 0, 0] if cos is None else [cos.data_ptr(), sin.data_ptr(),
+                                                          cos.stride(0) if cos.shape[0] > 1 else 0, cos.stride(1)]
+            _lib.check(_lib.load().carekv_rope_heads(q.data_ptr(), k.data_ptr(), v.data_ptr(), *ptr, B, T, Hq, Hkv, D,
+                                                     qo.data_ptr(), ko.data_ptr(), vo.data_ptr(),
+                                                     _lib.stream_ptr(q.device)), "carekv_rope_heads")
+            return qo, ko, vo
+        if cos is not None:
+            Q, K = _rope(Q, K, cos, sin)
+        return Q.to(F16).contiguous(), K.to(F16).contiguous(), V.to(F16).contiguous()
 
     def _out(self, O: Tensor, dtype) -> Tensor:
         """O (B, Hq, T, D) -> (B, T, model_dim) through W_O."""
@@ -216,11 +250,7 @@ class CAREKVLayer(nn.Module):
         if runs is not None:
             out = self._prefill_runs(cache, hidden, runs, sink_tokens, position_embeddings, token_start_abs, seqs)
             return out[0] if squeeze else out
-        Q, K, V = self._project(hidden)
-        if position_embeddings is not None:
-            cos, sin = position_embeddings
-            Q, K = _rope(Q, K, cos.to(Q.dtype), sin.to(Q.dtype))
-        Qh, Kh, Vh = Q.to(F16).contiguous(), K.to(F16).contiguous(), V.to(F16).contiguous()
+        Qh, Kh, Vh = self._heads(hidden, position_embeddings)
         hats = cache.write_prefill(self.layer_id, Kh, Vh, token_start_abs=token_start_abs,
                                    sink_tokens=sink_tokens, seqs=seqs)
         if mode == "fp":
@@ -265,14 +295,11 @@ class CAREKVLayer(nn.Module):
         if squeeze:
             hidden = hidden.unsqueeze(0)
         B = hidden.shape[0]
-        Q, K, V = self._project(hidden[:, -1:])
-        if position_embeddings is not None:
-            cos, sin = position_embeddings
-            Q, K = _rope(Q, K, cos.to(Q.dtype), sin.to(Q.dtype))
+        Q, K, V = self._heads(hidden[:, -1:], position_embeddings)
         seqs = list(range(B)) if seqs is None else list(seqs)
-        cache.append(self.layer_id, K[:, :, 0].to(F16), V[:, :, 0].to(F16), seqs=seqs)
+        cache.append(self.layer_id, K[:, :, 0], V[:, :, 0], seqs=seqs)
         correction, knobs = decode_read_mode(self.cfg, self.layer_id)
-        O = decode_attention(cache, self.layer_id, Q[:, :, 0].to(F16), seqs=seqs, correction=correction,
+        O = decode_attention(cache, self.layer_id, Q[:, :, 0], seqs=seqs, correction=correction,
                              knobs=knobs)  # (B, Hq, D)
         out = self._out(O.unsqueeze(2), hidden.dtype).to(hidden.dtype)  # (B, 1, model_dim)
         return out[0] if squeeze else out

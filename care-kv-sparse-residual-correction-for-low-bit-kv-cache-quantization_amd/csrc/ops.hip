@@ -173,6 +173,40 @@ __global__ __launch_bounds__(64) void write_base_kernel(carekv_arena A, long pg,
   if (lane == 0) A.valid[pg] = num_valid;
 }
 
+// A projected layer's heads, [b][t][h][d] -> [b][h][t][d], q and k rotated.
+// One thread per 4 dims of the lower half and their partners D/2 above: the
+// rotation, the head-major layout and the copies of q, k and v are one pass of
+// 8-byte loads and stores, where the elementwise form took ten launches with
+// their intermediate tensors.  Every product and sum is rounded to fp16 as
+// the elementwise form rounds it.
+__global__ __launch_bounds__(256) void rope_heads_kernel(const uint16_t* q, const uint16_t* k, const uint16_t* v,
+                                                         const uint16_t* cos, const uint16_t* sin, long cs_batch,
+                                                         long cs_row, int T, int Hq, int Hkv, int D, long n,
+                                                         uint16_t* qo, uint16_t* ko, uint16_t* vo) {
+  typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int per = D / 8, d = (int)(i % per) * 4, H = Hq + 2 * Hkv;
+  const long r = i / per;
+  const int h = (int)(r % H);
+  const long bt = r / H, b = bt / T, t = bt % T;
+  const bool isq = h < Hq, isk = !isq && h < Hq + Hkv;
+  const int nh = isq ? Hq : Hkv, hh = isq ? h : isk ? h - Hq : h - Hq - Hkv;
+  const uint16_t* x = (isq ? q : isk ? k : v) + (bt * nh + hh) * D + d;
+  uint16_t* y = (isq ? qo : isk ? ko : vo) + ((b * nh + hh) * T + t) * D + d;
+  const h4 x1 = *reinterpret_cast<const h4*>(x), x2 = *reinterpret_cast<const h4*>(x + D / 2);
+  h4 y1 = x1, y2 = x2;
+  if (cos && (isq || isk)) {
+    const long c = b * cs_batch + t * cs_row + d;
+    const h4 c1 = *reinterpret_cast<const h4*>(cos + c), c2 = *reinterpret_cast<const h4*>(cos + c + D / 2);
+    const h4 s1 = *reinterpret_cast<const h4*>(sin + c), s2 = *reinterpret_cast<const h4*>(sin + c + D / 2);
+    y1 = x1 * c1 + (-x2) * s1;
+    y2 = x2 * c2 + x1 * s2;
+  }
+  *reinterpret_cast<h4*>(y) = y1;
+  *reinterpret_cast<h4*>(y + D / 2) = y2;
+}
+
 }  // namespace carekv
 
 using namespace carekv;
@@ -282,4 +316,24 @@ extern "C" int carekv_write_base(const carekv_arena* arena, int32_t seq, int32_t
     CAREKV_CHECK_LAUNCH("write_base");
     return CAREKV_OK;
   });
+}
+
+extern "C" int carekv_rope_heads(const uint16_t* q, const uint16_t* k, const uint16_t* v, const uint16_t* cos,
+                                 const uint16_t* sin, int64_t cs_batch, int64_t cs_row, int32_t batch, int32_t seq_len,
+                                 int32_t n_heads, int32_t n_kv_heads, int32_t head_dim, uint16_t* qo, uint16_t* ko,
+                                 uint16_t* vo, void* stream) {
+  CAREKV_REQUIRE(q && k && v && qo && ko && vo && (!cos == !sin), "null argument");
+  CAREKV_REQUIRE(batch > 0 && seq_len > 0 && n_heads > 0 && n_kv_heads > 0, "counts must be positive");
+  CAREKV_REQUIRE(head_dim > 0 && head_dim % 8 == 0, "head_dim must be a multiple of 8");
+  uintptr_t bits = 0;
+  for (const void* p : {(const void*)q, (const void*)k, (const void*)v, (const void*)cos, (const void*)sin,
+                        (const void*)qo, (const void*)ko, (const void*)vo})
+    bits |= reinterpret_cast<uintptr_t>(p);
+  CAREKV_REQUIRE((bits & 7) == 0 && cs_batch % 4 == 0 && cs_row % 4 == 0, "operands must be 8-byte aligned");
+  const long n = (long)batch * seq_len * (n_heads + 2 * n_kv_heads) * (head_dim / 8);
+  CAREKV_REQUIRE(n < (1L << 31) * 256, "too many elements");
+  hipLaunchKernelGGL(rope_heads_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, q, k, v, cos,
+                     sin, cs_batch, cs_row, seq_len, n_heads, n_kv_heads, head_dim, n, qo, ko, vo);
+  CAREKV_CHECK_LAUNCH("rope_heads");
+  return CAREKV_OK;
 }

@@ -1046,10 +1046,28 @@ __global__ __launch_bounds__(256) void kivi_token_kernel(const uint16_t* __restr
 // Decode append for the fp16 side-buffer base: one wave per row; K per
 // channel over the one row (scale |k_d| / qmax), V per token
 // (layer.py:1037-1075, cache.py:820-838).
+// The open-page buffers' share of an append: the row's true values at its
+// offset (open_k NULL: not kept).
+struct OpenRows {
+  uint16_t* k;
+  uint16_t* v;
+};
+template <int D>
+__device__ __forceinline__ void keep_open_row(const OpenRows& op, const carekv_arena& A, const uint16_t* Kx,
+                                              const uint16_t* Vx, int row, int seq, int kvh, int off, int lane) {
+  if (!op.k) return;
+  const long at = (((long)seq * A.n_kv_heads + kvh) * kPage + off) * D;
+  for (int d = lane; d < D; d += 64) {
+    op.k[at + d] = Kx[(long)row * D + d];
+    op.v[at + d] = Vx[(long)row * D + d];
+  }
+}
+
 template <int D>
 __global__ __launch_bounds__(256) void append_hat_rows_kernel(carekv_arena A, const uint16_t* __restrict__ Kx,
                                                               const uint16_t* __restrict__ Vx,
-                                                              const int32_t* __restrict__ dest, int n_rows) {
+                                                              const int32_t* __restrict__ dest, int n_rows,
+                                                              OpenRows op) {
   constexpr int NG = D / 32;
   const int lane = threadIdx.x & 63;
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -1059,6 +1077,7 @@ __global__ __launch_bounds__(256) void append_hat_rows_kernel(carekv_arena A, co
   const int off = fresh ? 0 : A.valid[pg];
   if (off >= kPage) return;  // caller contract violated; never write past the page
   if (!code_pg_in(A, pg)) return;  // a page the code-page map does not hold: never written
+  keep_open_row<D>(op, A, Kx, Vx, row, seq, kvh, off, lane);
   const long cpg = code_pg(A, pg);
   uint16_t* krow = reinterpret_cast<uint16_t*>(A.kcodes) + (cpg * kPage + off) * D;
   uint16_t* vrow = reinterpret_cast<uint16_t*>(A.vcodes) + (cpg * kPage + off) * D;
@@ -1122,7 +1141,7 @@ template <int D, int BITS>
 __global__ __launch_bounds__(256) void append_rows_kernel(carekv_arena A, const uint16_t* __restrict__ Kx,
                                                           const uint16_t* __restrict__ Vx,
                                                           const int32_t* __restrict__ dest, int n_rows,
-                                                          CodedRows cr) {
+                                                          CodedRows cr, OpenRows op) {
   constexpr int NG = D / 32;
   constexpr int RB = row_bytes(D, BITS);
   constexpr int CB = 4 * BITS;
@@ -1133,6 +1152,7 @@ __global__ __launch_bounds__(256) void append_rows_kernel(carekv_arena A, const 
   const long pg = ((long)kvh * A.n_seq + seq) * A.max_pages + page;
   const int off = fresh ? 0 : A.valid[pg];
   if (off >= kPage) return;  // caller contract violated; never write past the page
+  keep_open_row<D>(op, A, Kx, Vx, row, seq, kvh, off, lane);
   const bool i8 = A.scale_mode == 1;
   // stored slots on the page (only a page with metadata can hold any)
   bool slots = false;
@@ -1585,13 +1605,97 @@ extern "C" int carekv_store_prefill(const carekv_arena* arena, const carekv_stor
 
 namespace {
 int append_any(const carekv_arena* arena, const uint16_t* k_rows, const uint16_t* v_rows, const int32_t* dest_dev,
-               int32_t n_rows, const CodedRows& cr, void* stream);
+               int32_t n_rows, const CodedRows& cr, const OpenRows& op, void* stream);
 }  // namespace
 
 extern "C" int carekv_append_rows(const carekv_arena* arena, const uint16_t* k_rows, const uint16_t* v_rows,
                                   const int32_t* dest_dev, int32_t n_rows, void* stream) {
   CAREKV_REQUIRE(k_rows && v_rows, "null argument");
-  return append_any(arena, k_rows, v_rows, dest_dev, n_rows, CodedRows{nullptr, nullptr, nullptr, nullptr}, stream);
+  return append_any(arena, k_rows, v_rows, dest_dev, n_rows, CodedRows{nullptr, nullptr, nullptr, nullptr},
+                    OpenRows{nullptr, nullptr}, stream);
+}
+
+extern "C" int carekv_append_rows_open(const carekv_arena* arena, const uint16_t* k_rows, const uint16_t* v_rows,
+                                       const int32_t* dest_dev, int32_t n_rows, uint16_t* open_k, uint16_t* open_v,
+                                       void* stream) {
+  CAREKV_REQUIRE(k_rows && v_rows && open_k && open_v, "null argument");
+  return append_any(arena, k_rows, v_rows, dest_dev, n_rows, CodedRows{nullptr, nullptr, nullptr, nullptr},
+                    OpenRows{open_k, open_v}, stream);
+}
+
+namespace carekv {
+// A work-group per (sequence, kv head): its open page's rows (the prompt's
+// partial last page, or zeros) and, with rescale_open, their group scales.
+template <int D, int BITS>
+__global__ __launch_bounds__(256) void open_rows_kernel(carekv_arena A, const uint16_t* __restrict__ K,
+                                                        const uint16_t* __restrict__ V,
+                                                        const int32_t* __restrict__ row_seq, int n_pages, int last,
+                                                        OpenRows op) {
+  constexpr int NG = D / 32;
+  const int b = blockIdx.x / A.n_kv_heads, kvh = blockIdx.x % A.n_kv_heads, seq = row_seq[b];
+  const long src = (((long)blockIdx.x * n_pages) + n_pages - 1) * kPage * D;  // the chunk's last page
+  if (op.k) {
+    const long at = ((long)seq * A.n_kv_heads + kvh) * kPage * D;
+    for (int i = threadIdx.x; i < kPage * D; i += 256) {
+      op.k[at + i] = last < kPage ? K[src + i] : 0;
+      op.v[at + i] = last < kPage ? V[src + i] : 0;
+    }
+  }
+  if (!A.rescale_open || last >= kPage) return;
+  const int t = threadIdx.x / (last * NG);  // K, then V
+  const int i = threadIdx.x % (last * NG);  // row, group
+  if (t > 1) return;
+  const uint16_t* x = (t ? V : K) + src + (long)i * 32;
+  float f[32];
+  int c[32];
+  for (int k = 0; k < 32; ++k) f[k] = h2f(x[k]);
+  const _Float16 s = quant_group<BITS>(f, c);
+  (t ? A.open_vscale : A.open_kscale)[((long)kvh * A.n_seq + seq) * kPage * NG + i] = half2bits(s);
+}
+
+__global__ __launch_bounds__(256) void reset_sequence_kernel(int32_t* valid, int8_t* has_meta, int32_t* k_slot,
+                                                             int32_t* v_slot, int32_t* next_slot, int n_lh, int n_seq,
+                                                             int P, int ncg, int nvb, int seq) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i < 2) next_slot[(long)seq * 2 + i] = 0;
+  if (i >= (long)n_lh * P) return;
+  const long pg = (i / P * n_seq + seq) * P + i % P;
+  valid[pg] = 0;
+  has_meta[pg] = 0;
+  for (int g = 0; g < ncg; ++g) k_slot[pg * ncg + g] = -1;
+  for (int v = 0; v < nvb; ++v) v_slot[pg * nvb + v] = -1;
+}
+}  // namespace carekv
+
+extern "C" int carekv_open_rows(const carekv_arena* arena, const uint16_t* K, const uint16_t* V, const int32_t* row_seq,
+                                int32_t n_rows, int32_t n_pages, int32_t last, uint16_t* open_k, uint16_t* open_v,
+                                void* stream) {
+  CAREKV_REQUIRE(arena && K && V && row_seq && (!open_k == !open_v), "null argument");
+  CAREKV_REQUIRE(check_arena(*arena), last_error_buf());
+  CAREKV_REQUIRE(n_pages >= 1 && last >= 1 && last <= kPage, "n_pages must be positive and last in 1..page_size");
+  if (n_rows <= 0) return CAREKV_OK;
+  // the base of a side-buffer arena plays no part: no scales are kept there
+  const int bits = arena->base_bits == 16 ? 2 : arena->base_bits;
+  return dispatch_db(arena->head_dim, bits, [&](auto d, auto b) {
+    hipLaunchKernelGGL((open_rows_kernel<decltype(d)::value, decltype(b)::value>),
+                       dim3((unsigned)n_rows * arena->n_kv_heads), dim3(256), 0, (hipStream_t)stream, *arena, K, V,
+                       row_seq, n_pages, last, OpenRows{open_k, open_v});
+    CAREKV_CHECK_LAUNCH("open_rows");
+    return CAREKV_OK;
+  });
+}
+
+extern "C" int carekv_reset_sequence(int32_t* valid, int8_t* has_meta, int32_t* k_slot, int32_t* v_slot,
+                                     int32_t* next_slot, int32_t n_layer_heads, int32_t n_seq, int32_t max_pages,
+                                     int32_t n_cgroups, int32_t n_vblocks, int32_t seq, void* stream) {
+  CAREKV_REQUIRE(valid && has_meta && k_slot && v_slot && next_slot, "null argument");
+  CAREKV_REQUIRE(n_layer_heads > 0 && max_pages > 0 && n_cgroups >= 0 && n_vblocks >= 0, "bad table shape");
+  CAREKV_REQUIRE(seq >= 0 && seq < n_seq, "seq out of range");
+  const long n = (long)n_layer_heads * max_pages;
+  hipLaunchKernelGGL(reset_sequence_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, valid,
+                     has_meta, k_slot, v_slot, next_slot, n_layer_heads, n_seq, max_pages, n_cgroups, n_vblocks, seq);
+  CAREKV_CHECK_LAUNCH("reset_sequence");
+  return CAREKV_OK;
 }
 
 extern "C" int carekv_append_coded_rows(const carekv_arena* arena, const int8_t* k_codes, const uint16_t* k_scale,
@@ -1599,12 +1703,13 @@ extern "C" int carekv_append_coded_rows(const carekv_arena* arena, const int8_t*
                                         int32_t n_rows, void* stream) {
   CAREKV_REQUIRE(k_codes && k_scale && v_codes && v_scale, "null argument");
   CAREKV_REQUIRE(arena && arena->base_bits != 16, "coded rows need a packed base");
-  return append_any(arena, nullptr, nullptr, dest_dev, n_rows, CodedRows{k_codes, k_scale, v_codes, v_scale}, stream);
+  return append_any(arena, nullptr, nullptr, dest_dev, n_rows, CodedRows{k_codes, k_scale, v_codes, v_scale},
+                    OpenRows{nullptr, nullptr}, stream);
 }
 
 namespace {
 int append_any(const carekv_arena* arena, const uint16_t* k_rows, const uint16_t* v_rows, const int32_t* dest_dev,
-               int32_t n_rows, const CodedRows& cr, void* stream) {
+               int32_t n_rows, const CodedRows& cr, const OpenRows& op, void* stream) {
   CAREKV_REQUIRE(arena && dest_dev, "null argument");
   if (n_rows <= 0) return CAREKV_OK;
   CAREKV_REQUIRE(check_arena(*arena), last_error_buf());
@@ -1617,16 +1722,16 @@ int append_any(const carekv_arena* arena, const uint16_t* k_rows, const uint16_t
   if (A.base_bits == 16) {
     if (A.head_dim == 64)
       hipLaunchKernelGGL(append_hat_rows_kernel<64>, dim3((n_rows + 3) / 4), dim3(256), 0, s, A, k_rows, v_rows,
-                         dest_dev, n_rows);
+                         dest_dev, n_rows, op);
     else
       hipLaunchKernelGGL(append_hat_rows_kernel<128>, dim3((n_rows + 3) / 4), dim3(256), 0, s, A, k_rows, v_rows,
-                         dest_dev, n_rows);
+                         dest_dev, n_rows, op);
     CAREKV_CHECK_LAUNCH("append_hat_rows");
     return CAREKV_OK;
   }
   return dispatch_db(A.head_dim, A.base_bits, [&](auto d, auto b) {
     hipLaunchKernelGGL((append_rows_kernel<decltype(d)::value, decltype(b)::value>), dim3((n_rows + 3) / 4),
-                       dim3(256), 0, s, A, k_rows, v_rows, dest_dev, n_rows, cr);
+                       dim3(256), 0, s, A, k_rows, v_rows, dest_dev, n_rows, cr, op);
     CAREKV_CHECK_LAUNCH("append_rows");
     return CAREKV_OK;
   });

@@ -236,6 +236,46 @@ int64_t carekv_store_workspace_bytes(const carekv_arena* arena, const carekv_sto
 int carekv_append_rows(const carekv_arena* arena, const uint16_t* k_rows, const uint16_t* v_rows,
                        const int32_t* dest_dev, int32_t n_rows, void* stream);
 
+/* carekv_append_rows that also keeps each appended row's true fp16 values in
+ * the sequence's open-page buffers open_k / open_v, fp16 [n_seq]
+ * [n_kv_heads][page_size][head_dim], at the row's page offset (no reference
+ * counterpart: what the streaming fill store reads). */
+int carekv_append_rows_open(const carekv_arena* arena, const uint16_t* k_rows, const uint16_t* v_rows,
+                            const int32_t* dest_dev, int32_t n_rows, uint16_t* open_k, uint16_t* open_v,
+                            void* stream);
+
+/* The open-page buffers after a prompt chunk (no reference counterpart):
+ * for each of n_rows sequences (row_seq: device int32 [n_rows]) and every kv
+ * head, with 0 < last < page_size the chunk's last page of K / V (fp16
+ * [n_rows][n_kv_heads][n_pages * page_size][head_dim], zero padded past its
+ * `last` rows), else zeros (last = page_size).  With rescale_open also the fp16
+ * group scales of its `last` rows (quantizer.py:31-55) into the arena's
+ * open_kscale / open_vscale.  open_k / open_v NULL: the scales only. */
+int carekv_open_rows(const carekv_arena* arena, const uint16_t* K, const uint16_t* V, const int32_t* row_seq,
+                     int32_t n_rows, int32_t n_pages, int32_t last, uint16_t* open_k, uint16_t* open_v,
+                     void* stream);
+
+/* Forget sequence slot `seq` (no reference counterpart: a reference cache
+ * holds one sequence): valid and has_meta to 0, the page slot tables to -1,
+ * the sequence's next slot ids to 0.  The tables are those of n_layer_heads =
+ * layers x kv heads rows, [n_layer_heads][n_seq][max_pages]. */
+int carekv_reset_sequence(int32_t* valid, int8_t* has_meta, int32_t* k_slot, int32_t* v_slot, int32_t* next_slot,
+                          int32_t n_layer_heads, int32_t n_seq, int32_t max_pages, int32_t n_cgroups,
+                          int32_t n_vblocks, int32_t seq, void* stream);
+
+/* The projections of a layer as its heads (layer.py:665-690, 996-1014): q
+ * fp16 [batch][seq_len][n_heads][head_dim] and k, v fp16 [batch][seq_len]
+ * [n_kv_heads][head_dim] -> [batch][heads][seq_len][head_dim], q and k under
+ * rotary position embeddings: half(half(x cos) + half(rot(x) sin)) with
+ * rot(x) = (-x[D/2:], x[:D/2]), transformers' apply_rotary_pos_emb in fp16.
+ * cos, sin: fp16 rows of head_dim values, row t of sequence b at
+ * b * cs_batch + t * cs_row elements (cs_batch 0: shared); NULL: no rotation.
+ * All pointers 8-byte aligned, cs_batch and cs_row multiples of 4. */
+int carekv_rope_heads(const uint16_t* q, const uint16_t* k, const uint16_t* v, const uint16_t* cos,
+                      const uint16_t* sin, int64_t cs_batch, int64_t cs_row, int32_t batch, int32_t seq_len,
+                      int32_t n_heads, int32_t n_kv_heads, int32_t head_dim, uint16_t* qo, uint16_t* ko, uint16_t* vo,
+                      void* stream);
+
 /* CAREKVCache.append_to_page (cache.py:656-701): rows already quantized by
  * the caller, int8 codes [n_rows][head_dim] and fp16 group scales
  * [n_rows][D/group], packed at (seq, kv_head, page, valid[pg]) with the
