@@ -255,6 +255,8 @@ class CAREKVCache:
         self._freed: Dict[Tuple[int, int], List[int]] = {}  # (seq, 0 K / 1 V) -> freed slot ids
         self._ws: Dict[str, torch.Tensor] = {}
         self._row_tables: Dict[tuple, torch.Tensor] = {}
+        self._row_indices: Dict[tuple, tuple] = {}
+        self._dest_tables: Dict[tuple, torch.Tensor] = {}
         self.status = _lib.StatusWatch()  # store calls' slot-overflow words, read without a sync
         # optional (start, end) torch.cuda.Event pair that write_prefill records
         # on the stream right before and after its store launches
@@ -488,16 +490,17 @@ class CAREKVCache:
         if k.dim() == 2:
             k, v = k.unsqueeze(0), v.unsqueeze(0)
         B, H, D = k.shape
-        seqs = list(range(B)) if seqs is None else list(seqs)
+        seqs = tuple(range(B)) if seqs is None else tuple(int(s) for s in seqs)
         # the row bookkeeping of every (sequence, kv head) at once: the open
         # page (the last page while it is not full) or a fresh one
         ps = cfg.page_size
-        sarr = np.asarray(seqs, dtype=np.int64)
-        hh, ss = np.arange(H)[None, :], sarr[:, None]
-        nxt = self.next_page[layer][:, sarr].T                              # (B, H)
-        vlast = self.valid_host[layer][hh, ss, np.maximum(nxt - 1, 0)]
-        fresh = ~((nxt > 0) & (vlast < ps))
-        if fresh.any():
+        sarr, hh, ss = self._row_index(seqs)
+        nxt = self.next_page[layer][hh, ss]                                  # (B, H)
+        pid = nxt - 1
+        offs = self.valid_host[layer][hh, ss, pid]
+        fresh = (nxt <= 0) | (offs >= ps)
+        any_fresh = bool(fresh.any())
+        if any_fresh:
             if self.kivi_packed:
                 over = fresh & (nxt - self.n_packed[sarr][:, None] >= self.tail_pages)
                 if over.any():
@@ -505,21 +508,21 @@ class CAREKVCache:
                     raise _lib.CarekvError(f"packed KIVI tail full: sequence {s_} has no fp16 tail page left "
                                            f"({self.tail_pages} per sequence, kivi_tail_pages)")
             assert (nxt[fresh] < cfg.max_pages).all(), "KV cache is full"
-        pid = np.where(fresh, nxt, nxt - 1)
-        if fresh.any():
+            pid = np.where(fresh, nxt, pid)
             # a fresh page starts at the row's token count (pages past the row's
             # next page hold no valid rows)
             tot = self.valid_host[layer][:, sarr, :].sum(-1).T               # (B, H)
             fb, fh = np.nonzero(fresh)
             self._token_start[layer, fh, sarr[fb], pid[fb, fh]] = tot[fb, fh]
             self.next_page[layer][:, sarr] += fresh.T
-        offs = self.valid_host[layer][hh, ss, pid]
-        self.valid_host[layer][hh, ss, pid] = offs + 1
-        dest = np.stack([np.broadcast_to(ss, (B, H)), np.broadcast_to(hh, (B, H)), pid, fresh],
-                        -1).reshape(B * H, 4).astype(np.int32)
-        fb, fh = np.nonzero(offs + 1 == ps)
-        filled = [(int(sarr[b_]), int(h_), int(pid[b_, h_])) for b_, h_ in zip(fb, fh)]  # the pages the appends fill
-        dest_d = to_device(dest, self.device)
+            offs = self.valid_host[layer][hh, ss, pid]
+        new = offs + 1
+        self.valid_host[layer][hh, ss, pid] = new
+        filled = []  # the pages the appends fill
+        if int(new.max(initial=0)) >= ps:
+            fb, fh = np.nonzero(new == ps)
+            filled = [(int(sarr[b_]), int(h_), int(pid[b_, h_])) for b_, h_ in zip(fb, fh)]
+        dest_d = self._append_dest(seqs, hh, ss, pid, fresh)
         kk = k.to(F16).contiguous().view(B * H, D)
         vv = v.to(F16).contiguous().view(B * H, D)
         lib = _lib.load()
@@ -531,6 +534,36 @@ class CAREKVCache:
                                                    _lib.stream_ptr(self.device)), "carekv_append_rows_open")
             if filled:
                 self._streaming_fill_store(layer, filled)
+
+    def _row_index(self, seqs: tuple):
+        """Index arrays of (sequence, kv head) rows: the sequences, and the kv
+        head and sequence of every cell of a (B, H) table."""
+        idx = self._row_indices.get(seqs)
+        if idx is None:
+            sarr = np.asarray(seqs, dtype=np.int64)
+            hh, ss = np.meshgrid(np.arange(self.cfg.num_kv_heads), sarr)
+            if len(self._row_indices) > 64:
+                self._row_indices.clear()
+            idx = self._row_indices[seqs] = (sarr, hh, ss)
+        return idx
+
+    def _append_dest(self, seqs: tuple, hh, ss, pid, fresh) -> torch.Tensor:
+        """carekv_append_rows' destinations (seq, kv_head, page, fresh), int32
+        [B * H][4] on the device.  The same for every layer of a token and for
+        the tokens of a page after its first, so the last tables are kept, per
+        stream (a table's upload is ordered on the stream that made it); a
+        captured call makes its own."""
+        def upload():
+            return to_device(np.stack((ss, hh, pid, fresh), -1).reshape(-1, 4).astype(np.int32), self.device)
+        if torch.cuda.is_current_stream_capturing():
+            return upload()
+        key = (_lib.stream_ptr(self.device), seqs, pid.tobytes(), fresh.tobytes())
+        t = self._dest_tables.get(key)
+        if t is None:
+            if len(self._dest_tables) > 64:
+                self._dest_tables.clear()
+            t = self._dest_tables[key] = upload()
+        return t
 
     def _streaming_fill_store(self, layer: int, filled):
         """Store the filled pages' residuals from their true rows against the
