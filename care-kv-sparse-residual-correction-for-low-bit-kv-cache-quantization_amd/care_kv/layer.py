@@ -107,7 +107,7 @@ class CAREKVLayer(nn.Module):
         cfg = self.cfg
         B, T, _ = hidden.shape
         Hq, Hkv, D = cfg.num_heads, cfg.num_kv_heads, cfg.head_dim
-        x = hidden.reshape(B * T, -1)  # (a 3-d product folds to this one on every call)
+        x = hidden.reshape(B * T, hidden.shape[-1])  # (a 3-d product folds to this one on every call)
         Q = (x @ self.W_Q.T).reshape(B, T, Hq, D).transpose(1, 2)
         K = (x @ self.W_K.T).reshape(B, T, Hkv, D).transpose(1, 2)
         V = (x @ self.W_V.T).reshape(B, T, Hkv, D).transpose(1, 2)
@@ -141,7 +141,7 @@ class CAREKVLayer(nn.Module):
     def _out(self, O: Tensor, dtype) -> Tensor:
         """O (B, Hq, T, D) -> (B, T, model_dim) through W_O."""
         B, Hq, T, D = O.shape
-        return (O.transpose(1, 2).reshape(B * T, Hq * D).to(self.W_O.dtype) @ self.W_O.T).reshape(B, T, -1)
+        return (O.transpose(1, 2).reshape(B * T, Hq * D).to(self.W_O.dtype) @ self.W_O.T).reshape(B, T, self.W_O.shape[0])
 
     @staticmethod
     def _key_runs(attention_mask: Optional[Tensor], B: int, T: int) -> Optional[list]:
