@@ -3,12 +3,14 @@
 // score and weight matrices are never materialised; the kernel returns O and,
 // optionally, the per-row log-sum-exp from which any weight can be rebuilt.
 //
-// One work-group per (block of 128 queries, query head, sequence), 4 waves of
-// 32 queries, on a one-dimensional grid whose order starts the longest
-// (latest) query blocks of every (sequence, head) first.  K and V tiles of 32
-// tokens are staged in LDS (double buffered, one barrier per tile; the next
-// tile's global loads are in flight while the current one is used); at
-// D = 128, 168 VGPRs and 35 KB of LDS, three work-groups share a CU:
+// One work-group per (block of 128 or 192 queries, query head, sequence), 4
+// waves of 32 or 48 queries, on a one-dimensional grid whose order starts the
+// longest (latest) query blocks first, a few heads of an XCD at a time: with
+// every head's blocks in flight their K/V passed the XCD's 4 MB L2 and the
+// tiles came from HBM.  K and V tiles of 32 tokens are staged in LDS (double
+// buffered, one barrier per tile; the next tile's global loads are in flight
+// while the current one is used); at D = 128, 168 VGPRs (235 with 48 queries
+// a wave) and 35 KB of LDS, three (two) work-groups share a CU:
 //   * S^T = K_hat Q^T: A = K tile rows (one 16-byte LDS read per lane and
 //     32-dim step), B = Q^T held in registers; lane l receives the scores of
 //     tokens 16tt + 4(l/16) + i for query l % 16 of a 16-query sub-block;
@@ -32,6 +34,7 @@
 // The K tile rows are padded to 2D + 16 bytes and the V tile rows to 2D + 32
 // bytes, so that each group of consecutive lanes of either LDS read pattern
 // touches every bank once.
+#include <algorithm>
 #include <cmath>
 
 #include "decode_page.h"
@@ -46,14 +49,17 @@ struct PrefillArgs {
   uint16_t* out;      // [B][Hq][T][D]
   float* lse;         // [B][Hq][T] natural log-sum-exp of the scaled scores, or null
   int B, Hq, Hkv, T, causal;
+  int group;          // heads of an XCD whose query blocks run together; 0: every head at once
   float sm_log2;      // sm_scale * log2(e)
 };
 
-template <int D>
-__global__ __launch_bounds__(256, 3) void prefill_attn_kernel(PrefillArgs a) {
+template <int D, int NQ>
+__global__ __launch_bounds__(256, NQ == 2 ? 3 : 2) void prefill_attn_kernel(PrefillArgs a) {
   constexpr int KT = 32;              // tokens per K/V tile
   constexpr int TT = KT / 16, NU = KT / 32;
-  constexpr int QB = 128;             // queries per work-group
+  constexpr int PS = NQ == 3 ? 3 : 2;
+  constexpr int QW = 16 * NQ;         // queries per wave
+  constexpr int QB = 4 * QW;          // and per work-group
   constexpr int KRS = 2 * D + 16;     // K tile row stride, bytes
   constexpr int VRS = 2 * D + 32;     // V tile row stride, bytes
   constexpr int KS = D / 32;          // 32-dim steps of the score product
@@ -67,25 +73,33 @@ __global__ __launch_bounds__(256, 3) void prefill_attn_kernel(PrefillArgs a) {
   typedef short short4_t __attribute__((ext_vector_type(4)));
   typedef __attribute__((address_space(3))) short4_t lds_short4;
 
-  // the longest (latest) query blocks of every (sequence, head) start first
+  // The longest (latest) query blocks start first.  Work-group ids go round the
+  // 8 XCDs; with a.group an XCD takes nh consecutive heads (the query heads of
+  // a kv head meet in one L2), a group of them at a time.
   const int nhb = a.Hq * a.B, nqb = gridDim.x / nhb;
-  const int qblk = nqb - 1 - (int)blockIdx.x / nhb, hb = (int)blockIdx.x % nhb;
+  int qblk = nqb - 1 - (int)blockIdx.x / nhb, hb = (int)blockIdx.x % nhb;
+  if (a.group) {
+    const int nh = nhb / 8, n = (int)blockIdx.x / 8;
+    const int first = n / (a.group * nqb) * a.group, cur = min(a.group, nh - first), r = n - first * nqb;
+    qblk = nqb - 1 - r / cur;
+    hb = (int)blockIdx.x % 8 * nh + first + r % cur;
+  }
   const int h = hb % a.Hq, b = hb / a.Hq;
   const int hk = h / (a.Hq / a.Hkv);
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, c16 = lane & 15;
   const int T = a.T;
-  const int q0 = qblk * QB, qw0 = q0 + 32 * w;
+  const int q0 = qblk * QB, qw0 = q0 + QW * w;
   const uint32_t span = (uint32_t)T * D * 2;
   const __amdgpu_buffer_rsrc_t rq = make_rsrc(a.q + ((long)b * a.Hq + h) * T * D, span);
   const __amdgpu_buffer_rsrc_t rk = make_rsrc(a.k + ((long)b * a.Hkv + hk) * T * D, span);
   const __amdgpu_buffer_rsrc_t rv = make_rsrc(a.v + ((long)b * a.Hkv + hk) * T * D, span);
 
   // Q^T operands: sub-block qb, step s -> query qw0 + 16 qb + c16, dims 32s + 8g ..
-  half8_t qf[2][KS];
+  half8_t qf[NQ][KS];
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb)
+  for (int qb = 0; qb < NQ; ++qb)
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
       const uint32_t qi = (uint32_t)(qw0 + 16 * qb + c16);
@@ -121,12 +135,15 @@ __global__ __launch_bounds__(256, 3) void prefill_attn_kernel(PrefillArgs a) {
     }
   };
 
-  float m_run[2] = {kLow, kLow}, l_run[2] = {0.f, 0.f};
-  float4_t o[2][DT];
+  float m_run[NQ], l_run[NQ];
+  float4_t o[NQ][DT];
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb)
+  for (int qb = 0; qb < NQ; ++qb) {
+    m_run[qb] = kLow;
+    l_run[qb] = 0.f;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) o[qb][dt] = float4_t{0.f, 0.f, 0.f, 0.f};
+  }
 
   load_tile(0);
   store_tile(0);
@@ -137,21 +154,21 @@ __global__ __launch_bounds__(256, 3) void prefill_attn_kernel(PrefillArgs a) {
     const char* kb = lds + (j & 1) * BUF;
     const char* vb = kb + KBUF;
     const int t0 = j * KT;
-    if (!a.causal || t0 <= qw0 + 31) {  // some query of the wave sees this tile
+    if (!a.causal || t0 <= qw0 + QW - 1) {  // some query of the wave sees this tile
       // ---- S^T = K_hat Q^T (raised wave priority over the MFMA blocks: a wave
       // with products to issue goes before the CU's other waves' softmax)
       __builtin_amdgcn_s_setprio(1);
-      float4_t s[TT][2];
+      float4_t s[TT][NQ];
 #pragma unroll
       for (int tt = 0; tt < TT; ++tt) {
-        s[tt][0] = float4_t{0.f, 0.f, 0.f, 0.f};
-        s[tt][1] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int qb = 0; qb < NQ; ++qb) s[tt][qb] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
           half8_t ak;
           *reinterpret_cast<uint4*>(&ak) = *reinterpret_cast<const uint4*>(kb + (16 * tt + c16) * KRS + (32 * ks + 8 * g) * 2);
-          s[tt][0] = mfma16x32(ak, qf[0][ks], s[tt][0]);
-          s[tt][1] = mfma16x32(ak, qf[1][ks], s[tt][1]);
+#pragma unroll
+          for (int qb = 0; qb < NQ; ++qb) s[tt][qb] = mfma16x32(ak, qf[qb][ks], s[tt][qb]);
         }
       }
       __builtin_amdgcn_s_setprio(0);
@@ -161,11 +178,11 @@ __global__ __launch_bounds__(256, 3) void prefill_attn_kernel(PrefillArgs a) {
       // exp2(x - m) is taken as exp2(fma(s, c, -m))
       const bool edge = (a.causal && t0 + KT - 1 > qw0) || t0 + KT > T;
       const float c = a.sm_log2;
-      float p[TT][2][4];
+      half8_t bp[NQ];
+      if (edge) {
 #pragma unroll
-      for (int qb = 0; qb < 2; ++qb) {
-        const int qi = qw0 + 16 * qb + c16;
-        if (edge) {
+        for (int qb = 0; qb < NQ; ++qb) {
+          const int qi = qw0 + 16 * qb + c16;
           // token 16 tt + i of the lane's rows is t0 + 4g + 16 tt + i; the
           // limits pass through an empty asm so that the compares stay on
           // this branch (most tiles are not edge tiles)
@@ -180,52 +197,54 @@ __global__ __launch_bounds__(256, 3) void prefill_attn_kernel(PrefillArgs a) {
             }
         }
       }
-      float ls[2];
-      auto weigh = [&]() {  // the weights and this lane's sums of them (its tokens; over the lane groups at the end)
+      // Two query columns at a time, so that their scores are dead when the
+      // next two's weights are made.
 #pragma unroll
-        for (int qb = 0; qb < 2; ++qb) {
-          ls[qb] = 0.f;
+      for (int q2 = 0; q2 < NQ; q2 += PS) {
+        float ls[PS];
+        auto weigh = [&]() {  // the weights and this lane's sums of them (its tokens; over the lane groups at the end)
 #pragma unroll
-          for (int tt = 0; tt < TT; ++tt)
+          for (int u = 0; u < PS; ++u) {
+            const int qb = q2 + u;
+            ls[u] = 0.f;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              p[tt][qb][i] = __builtin_amdgcn_exp2f(fmaf(s[tt][qb][i], c, -m_run[qb]));
-              ls[qb] += p[tt][qb][i];
+            for (int i = 0; i < 8; ++i) {
+              const float p = __builtin_amdgcn_exp2f(fmaf(s[i / 4][qb][i % 4], c, -m_run[qb]));
+              ls[u] += p;
+              bp[qb][i] = (_Float16)p;
             }
-        }
-      };
-      weigh();
-      // The reference maximum moves only when the weights outgrow it (a lane's
-      // sum over kSlack, so no weight passes it): most tiles need no maximum,
-      // no reduction over the lane groups and no rescale.  The first tile
-      // always comes here (m_run = kLow makes its sums infinite).
-      if (__builtin_expect(__any(ls[0] > kSlack || ls[1] > kSlack), 0)) {
-#pragma unroll
-        for (int qb = 0; qb < 2; ++qb) {
-          float mx = s[0][qb][0];
-#pragma unroll
-          for (int k = 1; k < 4 * TT; ++k) mx = fmaxf(mx, s[k / 4][qb][k % 4]);
-          const float m_new = fmaxf(m_run[qb], pair32_max(pair16_max(mx)) * c);
-          const float f = __builtin_amdgcn_exp2f(m_run[qb] - m_new);
-          m_run[qb] = m_new;
-          l_run[qb] *= f;
-#pragma unroll
-          for (int dt = 0; dt < DT; ++dt) o[qb][dt] *= f;
-        }
+          }
+        };
         weigh();
+        // The reference maximum moves only when the weights outgrow it (a lane's
+        // sum over kSlack, so no weight passes it): most tiles need no maximum,
+        // no reduction over the lane groups and no rescale.  The first tile
+        // always comes here (m_run = kLow makes its sums infinite).
+        bool over = ls[0] > kSlack;
+#pragma unroll
+        for (int u = 1; u < PS; ++u) over |= ls[u] > kSlack;
+        if (__builtin_expect(__any(over), 0)) {
+#pragma unroll
+          for (int qb = q2; qb < q2 + PS; ++qb) {
+            float mx = s[0][qb][0];
+#pragma unroll
+            for (int k = 1; k < 4 * TT; ++k) mx = fmaxf(mx, s[k / 4][qb][k % 4]);
+            const float m_new = fmaxf(m_run[qb], pair32_max(pair16_max(mx)) * c);
+            const float f = __builtin_amdgcn_exp2f(m_run[qb] - m_new);
+            m_run[qb] = m_new;
+            l_run[qb] *= f;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) o[qb][dt] *= f;
+          }
+          weigh();
+        }
+#pragma unroll
+        for (int u = 0; u < PS; ++u) l_run[q2 + u] += ls[u];
       }
-      l_run[0] += ls[0];
-      l_run[1] += ls[1];
       __builtin_amdgcn_s_setprio(1);
       // ---- O^T += V_hat^T P^T, 32 tokens per step
 #pragma unroll
       for (int u = 0; u < NU; ++u) {
-        half8_t bp[2];
-#pragma unroll
-        for (int qb = 0; qb < 2; ++qb)
-          bp[qb] = half8_t{(_Float16)p[2 * u][qb][0], (_Float16)p[2 * u][qb][1], (_Float16)p[2 * u][qb][2],
-                           (_Float16)p[2 * u][qb][3], (_Float16)p[2 * u + 1][qb][0], (_Float16)p[2 * u + 1][qb][1],
-                           (_Float16)p[2 * u + 1][qb][2], (_Float16)p[2 * u + 1][qb][3]};
         // source lane c16 of group g reads row 32u + 4g + c16/4 (and +16), dims 16dt + 4(c16%4) ..
         const __attribute__((address_space(3))) char* vrow =
             (const __attribute__((address_space(3))) char*)vb + (32 * u + 4 * g + (c16 >> 2)) * VRS + (c16 & 3) * 8;
@@ -236,8 +255,8 @@ __global__ __launch_bounds__(256, 3) void prefill_attn_kernel(PrefillArgs a) {
           half8_t av;
           __builtin_memcpy(&av, &v1, 8);
           __builtin_memcpy(reinterpret_cast<char*>(&av) + 8, &v2, 8);
-          o[0][dt] = mfma16x32(av, bp[0], o[0][dt]);
-          o[1][dt] = mfma16x32(av, bp[1], o[1][dt]);
+#pragma unroll
+          for (int qb = 0; qb < NQ; ++qb) o[qb][dt] = mfma16x32(av, bp[qb], o[qb][dt]);
         }
       }
     }
@@ -249,7 +268,7 @@ __global__ __launch_bounds__(256, 3) void prefill_attn_kernel(PrefillArgs a) {
 
   // ---- normalise and write (lane: query qw0 + 16qb + c16, dims 16dt + 4g ..)
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb) {
+  for (int qb = 0; qb < NQ; ++qb) {
     const float lt = pair32_sum(pair16_sum(l_run[qb]));
     const float inv = 1.f / lt;
     const int qi = qw0 + 16 * qb + c16;
@@ -295,12 +314,34 @@ extern "C" int carekv_prefill_attn(const carekv_prefill_params* pp, const uint16
   a.q = q; a.k = k; a.v = v; a.out = out; a.lse = lse;
   a.B = pp->batch; a.Hq = pp->n_heads; a.Hkv = pp->n_kv_heads; a.T = pp->seq_len; a.causal = pp->causal != 0;
   a.sm_log2 = pp->sm_scale * 1.4426950408889634f;
-  const long nblk = (long)((pp->seq_len + 127) / 128) * pp->n_heads * pp->batch;
+  const long hb = (long)pp->n_heads * pp->batch, T = pp->seq_len;
+  // D = 128: 48 queries a wave where the grid is at least 8 rounds of the GPU's
+  // 512 resident work-groups.  A tile's LDS reads then feed three query
+  // sub-blocks instead of two, for two work-groups a CU instead of three
+  // (4 x 40 heads, T = 8192: 2660 -> 2600 us; 8 x 32 / 8 heads, T = 3000: 635 ->
+  // 625 us).  Shorter grids lose more on their last round and their diagonal
+  // tiles (2 x 32 / 8 heads, T = 4096: 277 against 283 us; T = 1024: 65 against 73).
+  const bool wide = pp->head_dim == 128 && T >= 2048 && (T + 191) / 192 * hb >= 4096;
+  const int qb = wide ? 192 : 128;
+  const long nblk = (T + qb - 1) / qb * hb;
   CAREKV_REQUIRE(nblk < (1L << 31), "too many query blocks");
+  // Heads per XCD that run together: about 32768 of their queries, 2 2/3 rounds
+  // of the XCD's resident work-groups, so that a few heads' K/V tiles stay in
+  // its L2 and the longest blocks still start early enough; groups of equal
+  // size, since a small last one runs alone.  4 x 40 heads, T = 8192: 3210 us
+  // with every head at once, 2655-2740 in groups of 2 to 10, 3213 in one group;
+  // B = 8, 32 / 4 heads, T = 8192, D = 64: 2555 -> 2290 us.  Head counts that 8
+  // does not divide would load the XCDs unevenly.
+  if (hb % 8 == 0) {
+    const long nh = hb / 8, n_groups = std::max(1L, nh * T / 32768);
+    a.group = (int)((nh + n_groups - 1) / n_groups);
+  }
   const dim3 grid((unsigned)nblk);
   hipStream_t s = (hipStream_t)stream;
-  if (pp->head_dim == 128) hipLaunchKernelGGL(prefill_attn_kernel<128>, grid, dim3(256), 0, s, a);
-  else hipLaunchKernelGGL(prefill_attn_kernel<64>, grid, dim3(256), 0, s, a);
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, a); };
+  if (pp->head_dim == 64) go(prefill_attn_kernel<64, 2>);
+  else if (wide) go(prefill_attn_kernel<128, 3>);
+  else go(prefill_attn_kernel<128, 2>);
   CAREKV_CHECK_LAUNCH("prefill_attn");
   return CAREKV_OK;
 }
