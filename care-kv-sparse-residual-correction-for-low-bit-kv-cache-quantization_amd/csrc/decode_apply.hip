@@ -35,9 +35,9 @@ constexpr bool same_slot_order() {
 }
 
 // One page of the apply pass as loaded ahead of its use.
-template <int D, int BITS>
+template <int D, int BITS, bool K1>
 struct ApplyItem {
-  static constexpr int NWC = PageGeom<D, BITS>::NWC, NCG = D / 32, CH = D / 4;
+  static constexpr int NWC = PageGeom<D, BITS>::NWC, NCG = K1 ? 1 : D / 32, CH = D / 4;
   int p;               // page (wave-uniform)
   int meta;            // page metadata, one field per lane
   unsigned mk;         // selection mask byte of this lane's query (ln)
@@ -52,15 +52,23 @@ struct ApplyItem {
   uint32_t rv[CH / 8]; // V residual chunk of tile row ln (when its block is selected)
   uint32_t rvs;        // and its scale (fp16 bits)
   bool rsel;           // tile row ln holds a selected V block
+  int cg, vb;          // K1: the first stored K channel group and V block (-1: none; wave-uniform)
 };
 
 // 4 waves per SIMD (2 for the fp16 base, whose rows take twice the
 // registers): the register budget is capped at 128 (256) VGPRs.
-template <int D, int BITS, int SM>
+//
+// K1: k_cap = v_cap = 1, one K and one V slot a page can be selected (rank 0:
+// the first stored ones), so the searches for ranks over channel groups and
+// blocks go away: the pass is bound by the instructions of a page, and at
+// D = 64 over prompt rows it also needs 96 VGPRs instead of 105, five waves per
+// SIMD instead of four.  Prompt correction of 2048 rows, 32 / 4 heads: 585 ->
+// 550 us a call, the same bits.
+template <int D, int BITS, int SM, bool K1>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BITS == 16 ? 2 : 4, 8)))
 void decode_apply_kernel(carekv_arena A, DecodeArgs a) {
   using G = PageGeom<D, BITS>;
-  using Item = ApplyItem<D, BITS>;
+  using Item = ApplyItem<D, BITS, K1>;
   static_assert(same_slot_order<D, BITS>(), "V residual tile must use the V_hat slot order");
   constexpr int NT = G::NT, NCG = G::NCG, CH = G::CH, CHB = G::CHB, RB = G::RB;
   constexpr int VT_WORDS = kPage * G::VROW;
@@ -160,9 +168,18 @@ void decode_apply_kernel(carekv_arena A, DecodeArgs a) {
     const unsigned kb = m.mk & 15u, vb = m.mk >> 4;
     d.kany = 0; d.vany = 0;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
+    for (int r = 0; r < (K1 ? 1 : 4); ++r) {
       if (__any((kb >> r) & 1u)) d.kany |= 1u << r;
       if (__any((vb >> r) & 1u)) d.vany |= 1u << r;
+    }
+    if constexpr (K1) {
+      d.cg = -1; d.vb = -1;
+#pragma unroll
+      for (int c = NCG - 1; c >= 0; --c)
+        if (pm.ksl[c] >= 0) d.cg = c;
+#pragma unroll
+      for (int v = kVtb - 1; v >= 0; --v)
+        if (pm.vsl[v] >= 0) d.vb = v;
     }
     d.e01 = 0u; d.e23 = 0u; d.mref = 0.f;
     if (qv) {
@@ -176,18 +193,32 @@ void decode_apply_kernel(carekv_arena A, DecodeArgs a) {
       const int gi = (lj * CH) / 32;
       if constexpr (SM == 1) d.vsc = __builtin_amdgcn_raw_buffer_load_b8(rr.vs, vrow * NCG + gi, 0, 0);
       else d.vsc = __builtin_amdgcn_raw_buffer_load_b16(rr.vs, (vrow * NCG + gi) * 2, 0, 0);
-      int rk = 0;
+      if constexpr (K1) {
+        int slot = -1;
 #pragma unroll
-      for (int cg = 0; cg < NCG; ++cg) {
-        d.kr[cg] = 0u; d.krs[cg] = 0u;
-        if (pm.ksl[cg] < 0) continue;
-        if (rk < a.k_cap && ((d.kany >> rk) & 1u)) {
-          const long so = (long)seq * A.n_slots + pm.ksl[cg];
+        for (int c = NCG - 1; c >= 0; --c)
+          if (pm.ksl[c] >= 0) slot = pm.ksl[c];
+        d.kr[0] = 0u; d.krs[0] = 0u;
+        if (slot >= 0) {
+          const long so = (long)seq * A.n_slots + slot;
           const __amdgpu_buffer_rsrc_t r = make_rsrc(A.k_res + so * G::KSB, G::KSB);
-          d.kr[cg] = __builtin_amdgcn_raw_buffer_load_b32(r, ln * 16 + lj * 4, 0, 0);
-          d.krs[cg] = A.k_res_scale[so];
+          d.kr[0] = __builtin_amdgcn_raw_buffer_load_b32(r, ln * 16 + lj * 4, 0, 0);
+          d.krs[0] = A.k_res_scale[so];
         }
-        ++rk;
+      } else {
+        int rk = 0;
+#pragma unroll
+        for (int cg = 0; cg < NCG; ++cg) {
+          d.kr[cg] = 0u; d.krs[cg] = 0u;
+          if (pm.ksl[cg] < 0) continue;
+          if (rk < a.k_cap && ((d.kany >> rk) & 1u)) {
+            const long so = (long)seq * A.n_slots + pm.ksl[cg];
+            const __amdgpu_buffer_rsrc_t r = make_rsrc(A.k_res + so * G::KSB, G::KSB);
+            d.kr[cg] = __builtin_amdgcn_raw_buffer_load_b32(r, ln * 16 + lj * 4, 0, 0);
+            d.krs[cg] = A.k_res_scale[so];
+          }
+          ++rk;
+        }
       }
     }
     d.rsel = false;
@@ -195,11 +226,18 @@ void decode_apply_kernel(carekv_arena A, DecodeArgs a) {
       // tile row ln: block ln / 4, token ln % 4 of that block's slot
       const int vb_row = ln >> 2;
       int rrank = -1, rslot = -1, r2 = 0;
+      if constexpr (K1) {
+        rrank = d.vb == vb_row ? 0 : -1;
 #pragma unroll
-      for (int v = 0; v < kVtb; ++v) {
-        if (pm.vsl[v] < 0) continue;
-        if (v == vb_row) { rrank = r2; rslot = pm.vsl[v]; }
-        ++r2;
+        for (int v = kVtb - 1; v >= 0; --v)
+          if (pm.vsl[v] >= 0) rslot = pm.vsl[v];
+      } else {
+#pragma unroll
+        for (int v = 0; v < kVtb; ++v) {
+          if (pm.vsl[v] < 0) continue;
+          if (v == vb_row) { rrank = r2; rslot = pm.vsl[v]; }
+          ++r2;
+        }
       }
       d.rsel = rrank >= 0 && rrank < a.v_cap && ((d.vany >> rrank) & 1u) && 4 * vb_row < pm.nv;
       if (d.rsel) {
@@ -238,7 +276,14 @@ void decode_apply_kernel(carekv_arena A, DecodeArgs a) {
     }
     // ---- dS over the K slots this lane's query selected
     float wk[4] = {0.f, 0.f, 0.f, 0.f};
-    if (cur.kany) {
+    if constexpr (K1) {
+      if (cur.kany && cur.cg >= 0) {
+        const float4_t racc = kslot_dot_w(cur.kr[0], sqr, D, cur.cg, ln, lj);
+        const float rs = (kbits & 1u) ? h2f((uint16_t)cur.krs[0]) : 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) wk[i] = fmaf(racc[i], rs, wk[i]);
+      }
+    } else if (cur.kany) {
       int rk = 0;
 #pragma unroll
       for (int cg = 0; cg < NCG; ++cg) {
@@ -255,11 +300,15 @@ void decode_apply_kernel(carekv_arena A, DecodeArgs a) {
     }
     // ---- V block of this lane's tokens (4j .. 4j+3): stored slot rank
     int vrank = -1, rv = 0;
+    if constexpr (K1) {
+      vrank = cur.vb == lj ? 0 : -1;  // (no stored block is -1: no lane's)
+    } else {
 #pragma unroll
-    for (int vb = 0; vb < kVtb; ++vb) {
-      if (cm.vsl[vb] < 0) continue;
-      if (vb == lj) vrank = rv;
-      ++rv;
+      for (int vb = 0; vb < kVtb; ++vb) {
+        if (cm.vsl[vb] < 0) continue;
+        if (vb == lj) vrank = rv;
+        ++rv;
+      }
     }
     const bool vsel = vrank >= 0 && vrank < a.v_cap && ((vbits >> vrank) & 1u);
     float ck[4], cv[4];
@@ -424,8 +473,12 @@ int launch_decode_apply(const carekv_arena& A, const DecodeArgs& a, hipStream_t 
   // prefill rows read the prompt's fp16 K_hat / V_hat whatever the cache base
   const int bits = a.pf ? 16 : A.base_bits, smode = a.pf ? 0 : A.scale_mode;
   return dispatch_dbs16(A.head_dim, bits, smode, [&](auto d, auto bb, auto sm) {
-    hipLaunchKernelGGL((decode_apply_kernel<decltype(d)::value, decltype(bb)::value, decltype(sm)::value>), grid,
-                       dim3(256), 0, s, A, a);
+    if (a.k_cap == 1 && a.v_cap == 1)
+      hipLaunchKernelGGL((decode_apply_kernel<decltype(d)::value, decltype(bb)::value, decltype(sm)::value, true>),
+                         grid, dim3(256), 0, s, A, a);
+    else
+      hipLaunchKernelGGL((decode_apply_kernel<decltype(d)::value, decltype(bb)::value, decltype(sm)::value, false>),
+                         grid, dim3(256), 0, s, A, a);
     CAREKV_CHECK_LAUNCH("decode_apply");
     return CAREKV_OK;
   });
