@@ -491,10 +491,13 @@ class CAREKVCache:
             k, v = k.unsqueeze(0), v.unsqueeze(0)
         B, H, D = k.shape
         seqs = tuple(range(B)) if seqs is None else tuple(int(s) for s in seqs)
+        if len(seqs) != B or H > cfg.num_kv_heads:  # the kernel reads a destination per row of k and v
+            raise ValueError(f"append: k / v of {B} sequences x {H} kv heads for {len(seqs)} sequence slots of "
+                             f"{cfg.num_kv_heads} kv heads")
         # the row bookkeeping of every (sequence, kv head) at once: the open
         # page (the last page while it is not full) or a fresh one
         ps = cfg.page_size
-        sarr, hh, ss = self._row_index(seqs)
+        sarr, hh, ss = self._row_index(seqs, H)
         nxt = self.next_page[layer][hh, ss]                                  # (B, H)
         pid = nxt - 1
         offs = self.valid_host[layer][hh, ss, pid]
@@ -535,16 +538,16 @@ class CAREKVCache:
             if filled:
                 self._streaming_fill_store(layer, filled)
 
-    def _row_index(self, seqs: tuple):
+    def _row_index(self, seqs: tuple, H: int):
         """Index arrays of (sequence, kv head) rows: the sequences, and the kv
         head and sequence of every cell of a (B, H) table."""
-        idx = self._row_indices.get(seqs)
+        idx = self._row_indices.get((seqs, H))
         if idx is None:
             sarr = np.asarray(seqs, dtype=np.int64)
-            hh, ss = np.meshgrid(np.arange(self.cfg.num_kv_heads), sarr)
+            hh, ss = np.meshgrid(np.arange(H), sarr)
             if len(self._row_indices) > 64:
                 self._row_indices.clear()
-            idx = self._row_indices[seqs] = (sarr, hh, ss)
+            idx = self._row_indices[seqs, H] = (sarr, hh, ss)
         return idx
 
     def _append_dest(self, seqs: tuple, hh, ss, pid, fresh) -> torch.Tensor:
