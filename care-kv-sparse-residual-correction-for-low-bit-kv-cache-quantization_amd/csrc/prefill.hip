@@ -3,30 +3,32 @@
 // score and weight matrices are never materialised; the kernel returns O and,
 // optionally, the per-row log-sum-exp from which any weight can be rebuilt.
 //
-// One work-group per (block of 128 or 192 queries, query head, sequence), 4
-// waves of 32 or 48 queries, on a one-dimensional grid whose order starts the
-// longest (latest) query blocks first, a few heads of an XCD at a time: with
-// every head's blocks in flight their K/V passed the XCD's 4 MB L2 and the
-// tiles came from HBM.  K and V tiles of 32 tokens are staged in LDS (double
-// buffered, one barrier per tile; the next tile's global loads are in flight
-// while the current one is used); at D = 128, 168 VGPRs (235 with 48 queries
-// a wave) and 35 KB of LDS, three (two) work-groups share a CU:
+// One work-group per (block of 128 queries, query head, sequence), 4 waves of
+// 32 queries, on a one-dimensional grid whose order starts the longest (latest)
+// query blocks first, a few heads of an XCD at a time: with every head's blocks
+// in flight their K/V passed the XCD's 4 MB L2 and the tiles came from HBM.
+// K and V tiles of 32 tokens are staged in LDS (double buffered, one barrier per
+// tile; the next tile's global loads are in flight while the current one is
+// used); at D = 128, 160 VGPRs and 35 KB of LDS, three work-groups share a CU.
+// 48 queries a wave (218 VGPRs, two work-groups) measured the same (4 x 40 heads, T =
+// 8192: 2912 us against 2917; 8 x 32 / 8 heads, T = 3000: 692 against 686).
 //   * S^T = K_hat Q^T: A = K tile rows (one 16-byte LDS read per lane and
 //     32-dim step), B = Q^T held in registers; lane l receives the scores of
 //     tokens 16tt + 4(l/16) + i for query l % 16 of a 16-query sub-block;
 //   * the online softmax runs per query column in fp32 on base-2 logits
 //     (scores scaled by log2(e)/sqrt(D) after the fp32 product, as the
 //     reference divides the fp32 product by sqrt(D));
-//     The weights are exp2(x - m) with a reference maximum m that moves only
-//     when a tile's weights outgrow it by 2^8: the maximum, its reduction over
-//     the lane groups, the rescale factor and its test were a third of the
-//     loop's VALU work (of about 120 instructions a tile 66 are left),
-//     which bounds the kernel with its 16 exponentials a tile.  B = 4, 40
-//     heads, T = 8192, D = 128: 3613 -> 3279 us; B = 8, 32 / 4 heads, T = 2047,
-//     D = 64: 226 -> 189 us.  The fp16 weights keep 11 bits each, but the
-//     largest is no longer exactly 1, as in the reference, whose normalised
-//     weights are rounded wherever they fall: 2.7e-4 against 2.5e-4 from a
-//     64-bit evaluation, most of both the output's own rounding;
+//     Each lane compares its own 8 scores with the column's running maximum;
+//     only where one is larger are they reduced over the lane groups, the sums
+//     rescaled and the maximum moved.  Columns that keep theirs are multiplied
+//     by exactly 1, so that a row's bits depend on its own scores alone.  The
+//     reduction and the factor in every tile took 3506 us against 3402 at B = 4,
+//     40 heads, T = 8192, D = 128, and 216 against 208 at B = 8, 32 / 4 heads,
+//     T = 2047, D = 64 (before the grouped order below).  A maximum that lags
+//     behind the scores by up to 2^8 was faster still (2670 against 2890 us with
+//     that order), but it rounds the weights of a row's largest scores, which
+//     are exactly 1 here: the error against a 64-bit evaluation rose from
+//     2.58e-4 to 2.69e-4 (D = 64: 2.52e-4 to 2.63e-4);
 //   * O^T += V_hat^T P^T: the weights are already in the B layout (the 8 k
 //     values of a lane are tokens 4(l/16) + i of two 16-token tiles), and
 //     the A operand V_hat^T comes from the token-major V tile through the
@@ -53,11 +55,11 @@ struct PrefillArgs {
   float sm_log2;      // sm_scale * log2(e)
 };
 
-template <int D, int NQ>
-__global__ __launch_bounds__(256, NQ == 2 ? 3 : 2) void prefill_attn_kernel(PrefillArgs a) {
+template <int D>
+__global__ __launch_bounds__(256, 3) void prefill_attn_kernel(PrefillArgs a) {
   constexpr int KT = 32;              // tokens per K/V tile
   constexpr int TT = KT / 16, NU = KT / 32;
-  constexpr int PS = NQ == 3 ? 3 : 2;
+  constexpr int NQ = 2;               // 16-query sub-blocks of a wave
   constexpr int QW = 16 * NQ;         // queries per wave
   constexpr int QB = 4 * QW;          // and per work-group
   constexpr int KRS = 2 * D + 16;     // K tile row stride, bytes
@@ -67,7 +69,6 @@ __global__ __launch_bounds__(256, NQ == 2 ? 3 : 2) void prefill_attn_kernel(Pref
   constexpr int KBUF = KT * KRS, VBUF = KT * VRS, BUF = KBUF + VBUF;
   constexpr int CHR = D / 8;          // 16-byte chunks per row
   constexpr int NCH = 2 * KT * CHR / 256;  // chunks a thread stages per tile
-  constexpr float kSlack = 256.f;     // weights up to 2^8, far inside fp16
   constexpr float kLow = -1e30f;      // below any score; finite, so that a masked score's weight is 0 from the first tile
   __shared__ __align__(16) char lds[2 * BUF];
   typedef short short4_t __attribute__((ext_vector_type(4)));
@@ -197,49 +198,43 @@ __global__ __launch_bounds__(256, NQ == 2 ? 3 : 2) void prefill_attn_kernel(Pref
             }
         }
       }
-      // Two query columns at a time, so that their scores are dead when the
-      // next two's weights are made.
+      // A column's maximum moves where one of its own lanes holds a larger
+      // score: only such a tile reduces it over the lane groups and rescales
+      // (the first always does).  Columns of the wave that keep theirs get a
+      // factor of exactly 1, so a row's bits do not depend on its neighbours.
+      float mx[NQ];
+      bool over[NQ], any_over = false;
 #pragma unroll
-      for (int q2 = 0; q2 < NQ; q2 += PS) {
-        float ls[PS];
-        auto weigh = [&]() {  // the weights and this lane's sums of them (its tokens; over the lane groups at the end)
+      for (int qb = 0; qb < NQ; ++qb) {
+        mx[qb] = -INFINITY;  // a chain of three-operand maxima over the lane's 8 scores
 #pragma unroll
-          for (int u = 0; u < PS; ++u) {
-            const int qb = q2 + u;
-            ls[u] = 0.f;
+        for (int k = 0; k < 4 * TT; k += 2) mx[qb] = fmaxf(fmaxf(mx[qb], s[k / 4][qb][k % 4]), s[k / 4][qb][k % 4 + 1]);
+        over[qb] = mx[qb] * c > m_run[qb];
+        any_over |= over[qb];
+      }
+      if (__any(any_over)) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-              const float p = __builtin_amdgcn_exp2f(fmaf(s[i / 4][qb][i % 4], c, -m_run[qb]));
-              ls[u] += p;
-              bp[qb][i] = (_Float16)p;
-            }
-          }
-        };
-        weigh();
-        // The reference maximum moves only when the weights outgrow it (a lane's
-        // sum over kSlack, so no weight passes it): most tiles need no maximum,
-        // no reduction over the lane groups and no rescale.  The first tile
-        // always comes here (m_run = kLow makes its sums infinite).
-        bool over = ls[0] > kSlack;
+        for (int qb = 0; qb < NQ; ++qb) {
+          if (!__any(over[qb])) continue;
+          const float m_new = fmaxf(m_run[qb], pair32_max(pair16_max(mx[qb])) * c);
+          const float f = __builtin_amdgcn_exp2f(m_run[qb] - m_new);
+          m_run[qb] = m_new;
+          l_run[qb] *= f;
 #pragma unroll
-        for (int u = 1; u < PS; ++u) over |= ls[u] > kSlack;
-        if (__builtin_expect(__any(over), 0)) {
-#pragma unroll
-          for (int qb = q2; qb < q2 + PS; ++qb) {
-            float mx = s[0][qb][0];
-#pragma unroll
-            for (int k = 1; k < 4 * TT; ++k) mx = fmaxf(mx, s[k / 4][qb][k % 4]);
-            const float m_new = fmaxf(m_run[qb], pair32_max(pair16_max(mx)) * c);
-            const float f = __builtin_amdgcn_exp2f(m_run[qb] - m_new);
-            m_run[qb] = m_new;
-            l_run[qb] *= f;
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt) o[qb][dt] *= f;
-          }
-          weigh();
+          for (int dt = 0; dt < DT; ++dt) o[qb][dt] *= f;
         }
+      }
+      // the weights, and this lane's sums of them (its tokens; over the lane groups at the end)
 #pragma unroll
-        for (int u = 0; u < PS; ++u) l_run[q2 + u] += ls[u];
+      for (int qb = 0; qb < NQ; ++qb) {
+        float ls = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float p = __builtin_amdgcn_exp2f(fmaf(s[i / 4][qb][i % 4], c, -m_run[qb]));
+          ls += p;
+          bp[qb][i] = (_Float16)p;
+        }
+        l_run[qb] += ls;
       }
       __builtin_amdgcn_s_setprio(1);
       // ---- O^T += V_hat^T P^T, 32 tokens per step
@@ -315,33 +310,23 @@ extern "C" int carekv_prefill_attn(const carekv_prefill_params* pp, const uint16
   a.B = pp->batch; a.Hq = pp->n_heads; a.Hkv = pp->n_kv_heads; a.T = pp->seq_len; a.causal = pp->causal != 0;
   a.sm_log2 = pp->sm_scale * 1.4426950408889634f;
   const long hb = (long)pp->n_heads * pp->batch, T = pp->seq_len;
-  // D = 128: 48 queries a wave where the grid is at least 8 rounds of the GPU's
-  // 512 resident work-groups.  A tile's LDS reads then feed three query
-  // sub-blocks instead of two, for two work-groups a CU instead of three
-  // (4 x 40 heads, T = 8192: 2660 -> 2600 us; 8 x 32 / 8 heads, T = 3000: 635 ->
-  // 625 us).  Shorter grids lose more on their last round and their diagonal
-  // tiles (2 x 32 / 8 heads, T = 4096: 277 against 283 us; T = 1024: 65 against 73).
-  const bool wide = pp->head_dim == 128 && T >= 2048 && (T + 191) / 192 * hb >= 4096;
-  const int qb = wide ? 192 : 128;
-  const long nblk = (T + qb - 1) / qb * hb;
+  const long nblk = (T + 127) / 128 * hb;
   CAREKV_REQUIRE(nblk < (1L << 31), "too many query blocks");
   // Heads per XCD that run together: about 32768 of their queries, 2 2/3 rounds
   // of the XCD's resident work-groups, so that a few heads' K/V tiles stay in
-  // its L2 and the longest blocks still start early enough; groups of equal
-  // size, since a small last one runs alone.  4 x 40 heads, T = 8192: 3210 us
-  // with every head at once, 2655-2740 in groups of 2 to 10, 3213 in one group;
-  // B = 8, 32 / 4 heads, T = 8192, D = 64: 2555 -> 2290 us.  Head counts that 8
-  // does not divide would load the XCDs unevenly.
+  // its L2 and the longest blocks still start early enough (the last group has
+  // the heads that are left).  4 x 40 heads, T = 8192: 2894 us against
+  // 3402 with every head at once; B = 8, 32 / 4 heads, D = 64: 2657 against 2840
+  // at T = 8192, 194 against 208 at T = 2047.  Head counts that 8 does not divide
+  // would load the XCDs unevenly and keep every head at once.
   if (hb % 8 == 0) {
     const long nh = hb / 8, n_groups = std::max(1L, nh * T / 32768);
     a.group = (int)((nh + n_groups - 1) / n_groups);
   }
   const dim3 grid((unsigned)nblk);
   hipStream_t s = (hipStream_t)stream;
-  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, a); };
-  if (pp->head_dim == 64) go(prefill_attn_kernel<64, 2>);
-  else if (wide) go(prefill_attn_kernel<128, 3>);
-  else go(prefill_attn_kernel<128, 2>);
+  if (pp->head_dim == 128) hipLaunchKernelGGL(prefill_attn_kernel<128>, grid, dim3(256), 0, s, a);
+  else hipLaunchKernelGGL(prefill_attn_kernel<64>, grid, dim3(256), 0, s, a);
   CAREKV_CHECK_LAUNCH("prefill_attn");
   return CAREKV_OK;
 }

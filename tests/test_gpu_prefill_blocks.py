@@ -1,7 +1,6 @@
-"""The prefill attention's block orders and widths against a plain fp32 product with an
-fp64 softmax:
-48 queries a wave (D = 128, long grids) with a ragged last block, head groups
-of unequal size, one group, and a head count that 8 does not divide.
+"""The prefill attention's block orders against a plain fp32 product with an
+fp64 softmax: head groups of unequal size with a ragged last block, one group,
+and a head count that 8 does not divide.
 
 Bars: the output within 2^-10 sum_t a_t |v_t| (two fp16 roundings of a weight)
 plus one fp16 ulp; the log-sum-exp within 2^-21 (|lse| + 8)."""
@@ -14,8 +13,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("B,Hq,Hkv,T,D,causal", [
-    (10, 40, 4, 2050, 128, True),    # 11 blocks of 192 x 400 heads; groups of 17, 17 and 16 heads
-    (12, 32, 4, 2113, 128, False),   # 48 queries a wave without the causal skip
+    (10, 40, 4, 2050, 128, True),    # ragged blocks; groups of 17, 17 and 16 heads
+    (12, 32, 4, 2113, 128, False),   # groups without the causal skip
     (3, 40, 5, 5000, 64, True),      # groups of 8 and 7 heads
     (2, 16, 2, 193, 128, True),      # one group
     (1, 12, 12, 129, 64, True),      # 12 heads: every head at once

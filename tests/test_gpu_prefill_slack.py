@@ -1,6 +1,5 @@
-"""The prefill attention's reference maximum, which moves only when a tile's
-weights outgrow it: scores that rise tile by tile (below and above the slack of
-2^8), one late peak, falling scores, and a first tile that is mostly masked,
+"""The prefill attention's running maximum, which is reduced only in tiles that
+hold a larger score: scores that rise tile by tile, in steps or slowly, one late peak, falling scores, and a first tile that is mostly masked,
 against an fp64 evaluation.
 
 Bars: the output within 2^-10 sum_t a_t |v_t| (two fp16 roundings of a weight)
