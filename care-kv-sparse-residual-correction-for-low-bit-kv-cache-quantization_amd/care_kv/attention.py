@@ -141,21 +141,22 @@ def decode_read_mode(cfg: CacheConfig, layer: int):
     return any_read_budget(cfg), knobs
 
 
-def default_split_pages(max_pages: int, rows: int, step: int = 16) -> int:
+def default_split_pages(max_pages: int, rows: int, step: int = 16, short_splits: int = 16) -> int:
     """Pages per work-group of the streaming pass, a multiple of ``step``
     (16: 4 waves x 4-page windows of the 4-query-head kernel; 4 where the
     kernel takes a page per wave): long enough that each wave's start-up (q
     staging, the first window's loads, the split merge) spreads over several
     windows -- half a row, at most 256 pages -- and short enough that the grid
     keeps at least CAREKV_DECODE_MIN_WGS (default 1024: four per CU)
-    work-groups."""
+    work-groups.  A row takes at most ``short_splits`` splits of fewer than
+    16 pages: each later pass of a row walks the partials of all its splits."""
     min_wgs = max(1, int(os.environ.get("CAREKV_DECODE_MIN_WGS", "1024")))
     P, R = max(1, max_pages), max(1, rows)
     if P * R > 32 * min_wgs:  # the grid is full either way, and fewer partials keep the workspace small
         step = max(step, 16)
     sp = max(step, min(256, -(-P // 2), (P * R) // min_wgs))
     if sp < 16:  # shorter splits pay for their partials only where they spread over idle CUs
-        sp = max(step, min(16, 2 * P * R // min_wgs))
+        sp = max(step, min(16, max(2 * P * R // min_wgs, -(-P // short_splits))))
     return (sp + step - 1) // step * step
 
 
@@ -287,12 +288,19 @@ def decode_attention(cache: CAREKVCache, layer: int, q: torch.Tensor, seqs: Opti
     short = False
     if split_pages is None:
         # more than 4 query heads per kv head, or fp16 pages: the kernel takes a
-        # page per wave, so rows too few to fill the GPU split down to 4 pages
-        # (4 rows of 32 pages: 27.9 us a step against 38.1 with 16-page splits;
-        # 128 rows of 144 pages: 66.0 us with 20 against 73 with 32; 32 rows of
-        # 250 pages keep 16: 58 us against 60 with 8)
+        # page per wave, so rows too few to fill the GPU split down to 4 pages.
+        # D = 64, 8 queries, 4 / 8 / 16 pages a split: 4 rows of 32 pages 27.6 /
+        # 30.3 / 35.4 us a step, of 128 pages 38.4 / 38.1 / 41.6, of 512 pages
+        # 68.2 / 52.7 / 49.9, of 1024 pages 110 / 76 / 62 (hence at most 16
+        # splits); 64 rows of 64 pages 40.0 / 37.2 / 40.7, of 256 pages 73.6 /
+        # 63.4 / 59.3.  The sketch proxy reads every split's O partial in every
+        # work-group, so its rows take at most 8 (2 rows, D = 128, 8 queries: 64
+        # pages 62.5 / 60.0 / 64.6, 128 pages 78.3 / 68.6 / 70.6, 2048 pages 8 / 16
+        # / 32 a split 347 / 217 / 166).
         page_wave = cfg.num_heads > 4 * cfg.num_kv_heads or (cache.hat and not cache.kivi_packed)
-        split_pages = default_split_pages(max_np, B * cfg.num_kv_heads, step=4 if page_wave else 16)
+        sketch = correction and not knobs.kscore_live
+        split_pages = default_split_pages(max_np, B * cfg.num_kv_heads, step=4 if page_wave else 16,
+                                          short_splits=8 if sketch else 16)
         short = page_wave
     dp = _read_params(cache, layer, knobs, batch=B, n_heads=Hq, correction=correction, split_pages=split_pages,
                       max_pages=max_np, seq_ptr=meta[0].data_ptr(), np_ptr=meta[1].data_ptr())
