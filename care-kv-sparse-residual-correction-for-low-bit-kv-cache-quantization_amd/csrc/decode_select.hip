@@ -1134,14 +1134,18 @@ int launch_decode_select(const carekv_arena& A, const DecodeArgs& a, hipStream_t
   const bool k1 = a.k_cap == 1 && a.v_cap == 1;
   // rows of at most 256 pages, and enough query columns to fill the GPU with
   // waves (or short rows, where the work-group form's fixed cost dominates):
-  // a wave per query.  CAREKV_SELECT_WAVE=0 keeps the work-group form, =2
-  // takes the wave form for every row it covers.
+  // a wave per query.  With several slots a page a lane's chain is longer: the
+  // wave form takes prompt rows, most of them shorter than the longest (2048
+  // rows, 2K + 4V: 988 -> 775 us a call), and decode rows of at most 64 pages in
+  // 2048 columns (2K + 4V, D = 128: 92 -> 88 us a step; of 94 pages 121 -> 122, of
+  // 250 pages 215 -> 225; 32 columns of 13 pages 42 -> 44).  CAREKV_SELECT_WAVE=0
+  // keeps the work-group form, =2 takes the wave form for every row it covers.
   const char* env = getenv("CAREKV_SELECT_WAVE");
   const int wmode = env ? env[0] - '0' : 1;
   const long cols = (long)pairs * a.GQ;
   if (wmode != 0 && a.correction && !px && (a.policy == 0 || a.policy == 1) && !a.adaptive_score && a.Pmax <= 256 &&
       a.nsplit <= 256 && a.F == 2 + 4 * a.k_cap + a.v_cap && a.k_cap <= A.head_dim / 32 && a.v_cap <= kVtb &&
-      (wmode == 2 || cols >= 2048 || a.Pmax <= 64)) {
+      (wmode == 2 || (k1 ? cols >= 2048 || a.Pmax <= 64 : a.pf || (cols >= 2048 && a.Pmax <= 64)))) {
     const int ngq = (a.GQ + 3) / 4;
     const dim3 gw(((pairs + kXcd - 1) / kXcd) * kXcd * ngq);
     auto wave = [&](auto d) {
