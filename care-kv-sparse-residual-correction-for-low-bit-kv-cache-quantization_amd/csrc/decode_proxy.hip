@@ -16,12 +16,16 @@
 // dequantises V_hat; afterwards token m of query 4 k + j.  The distances are
 // ||V_hat_t||^2 + ||O||^2 - 2 V_hat_t . O on 16x16x32 MFMAs: the dequantised
 // registers are the B operand as they stand (the dims in the codes' pair
-// order), the A operand's rows 4 j and 4 j + 1 hold query 4 k + j of O split in
-// fp16 hi + lo at a power of two of its own (22 bits of its largest element),
-// and the norms are the diagonal of V_hat V_hat^T.  Where that cancels (a token
-// near O_base) the page takes the differences themselves.  A page of 4 queries
-// costs about 200 VALU operations and 8 MFMAs; the differences alone took 384
-// VALU and 128 LDS reads.  A page's loads are issued while the page before it
+// order), the A operand's rows 4 j .. 4 j + 2 hold query 4 k + j of O in three
+// fp16 parts at a power of two of its own (33 bits of its largest element, the
+// whole fp32 value), and the norms are the diagonal of V_hat V_hat^T.  Where the
+// sum loses more than a third of its terms (a token near O_base), or is not
+// finite, the pair takes the differences themselves, so that the distances keep
+// the differences' error against 64 bits (D = 128, rms: V around zero 4.7e-8,
+// differences 4.8e-8; around one deviation 5.3e-8 both, 6.5e-8 where it may
+// lose half; around 3.5 deviations 7.6e-8 both, 4.3e-7 where it may lose 31/32).  A page of 4 queries costs about
+// 200 VALU operations and 8 MFMAs; the differences alone took 384 VALU and 128
+// LDS reads.  A page's loads are issued while the page before it
 // is worked on, and the split statistics are read by lanes side by side (a thread
 // per query walked them before, two memory round trips a split).  Measured at
 // 8 sequences x 8 kv heads x 8185 tokens, INT4, D = 128, 4 queries:
@@ -56,6 +60,7 @@ __global__ __launch_bounds__(256) void decode_proxy_kernel(carekv_arena A, Decod
   constexpr int KS = CH / 8;                  // MFMA steps (8 dims of each lane group)
   constexpr float kEps = 1e-6f;               // residual_router.py:34
   constexpr float kLn2 = 0.693147180559945f;  // margins back from base-2 logits
+  constexpr float kCancel = 1.5f;             // the expansion's terms are at most this multiple of the distance
   __shared__ float s_o[16 * D];               // O_base [query][dim]
   __shared__ float s_M[16], s_L[16], s_Mp[16], s_oo[16], s_up[16], s_dn[16];
 
@@ -137,12 +142,13 @@ __global__ __launch_bounds__(256) void decode_proxy_kernel(carekv_arena A, Decod
     }
   }
   __syncthreads();
-  // A operands: row ln = 4 (query) + part (hi, lo, zero, zero), this lane's dims in the codes' pair order
+  // A operands: row ln = 4 (query) + part (high, middle, low, zero), this lane's dims in the codes' pair order
   half8_t op[NG][KS];
 #pragma unroll
   for (int k = 0; k < NG; ++k) {
     const int qq = 4 * k + (ln >> 2);
-    const bool on = qq < GQ && (ln & 3) < 2;
+    const int part = ln & 3;
+    const bool on = qq < GQ && part < 3;
     const float up = on ? s_up[qq] : 0.f;
     const float* o = s_o + (on ? qq : 0) * D + lj * CH;
 #pragma unroll
@@ -150,8 +156,9 @@ __global__ __launch_bounds__(256) void decode_proxy_kernel(carekv_arena A, Decod
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         const float x = on ? o[u ? PB::T.b[i] : PB::T.a[i]] * up : 0.f;
-        const _Float16 hi = (_Float16)x, lo = (_Float16)(x - (float)hi);
-        op[k][i / 4][2 * (i % 4) + u] = ln & 1 ? lo : hi;
+        const _Float16 hi = (_Float16)x, mid = (_Float16)(x - (float)hi);
+        const _Float16 lo = (_Float16)((x - (float)hi) - (float)mid);
+        op[k][i / 4][2 * (i % 4) + u] = part == 0 ? hi : part == 1 ? mid : lo;
       }
     }
   }
@@ -223,8 +230,9 @@ __global__ __launch_bounds__(256) void decode_proxy_kernel(carekv_arena A, Decod
       for (int ks = 0; ks < KS; ++ks) vo = mfma16x32(op[k][ks], vb[ks], vo);
       const bool in = qq < GQ && ln < nv;
       const float sum = vv + s_oo[in ? qq : 0];
-      float d2 = fmaf(-2.f, (vo[0] + vo[1]) * s_dn[in ? qq : 0], sum);
-      if (__any(in && d2 * 32.f < sum)) {
+      float d2 = fmaf(-2.f, (vo[0] + (vo[1] + vo[2])) * s_dn[in ? qq : 0], sum);
+      const bool near = in && !(d2 * kCancel >= sum);  // (or not finite)
+      if (__any(near)) {
         // ||V_hat_t - O_q||^2 for queries q0 .. q0+3; row j keeps query q0 + j
 #pragma unroll 1
         for (int u = 0; u < 4; ++u) {
@@ -239,7 +247,7 @@ __global__ __launch_bounds__(256) void decode_proxy_kernel(carekv_arena A, Decod
             acc = fmaf(d1, d1, acc);
           }
           const float tot = col_sum(acc);
-          if (lj == u) d2 = tot;
+          if (lj == u && near) d2 = tot;
         }
       }
       float at = 0.f, bt = 0.f, vt = 0.f;
@@ -272,7 +280,11 @@ int launch_decode_proxy(const carekv_arena& A, const DecodeArgs& a, hipStream_t 
   }
   return dispatch_dbs16(A.head_dim, A.base_bits, A.scale_mode, [&](auto d, auto bb, auto sm) {
     constexpr int D = decltype(d)::value, BITS = decltype(bb)::value, SM = decltype(sm)::value;
-    // one group of four queries costs a quarter of the operand registers
+    // one group of four queries costs a quarter of the operand registers (D =
+    // 128: 114-122 VGPRs, four waves per SIMD, against 185-194, two; the
+    // differences alone took 82).  Both beat the differences: 8 sequences of 8185
+    // tokens, 32 / 8 heads 143 -> 106 us a step, 40 / 8 183 -> 170, 16 / 2 178 ->
+    // 120, 32 / 2 253 -> 160; 32 / 2 heads, D = 64, 176 -> 122
     if (a.GQ <= 4) hipLaunchKernelGGL((decode_proxy_kernel<D, BITS, SM, 1>), grid, dim3(256), 0, s, A, a);
     else hipLaunchKernelGGL((decode_proxy_kernel<D, BITS, SM, 4>), grid, dim3(256), 0, s, A, a);
     CAREKV_CHECK_LAUNCH("decode_proxy");
