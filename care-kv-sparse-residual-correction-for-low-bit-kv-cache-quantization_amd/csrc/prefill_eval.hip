@@ -95,6 +95,13 @@ __device__ __forceinline__ half8_t minus(const half8_t& x, const half8_t& y) {
   }
   return r;
 }
+// Its infinite and NaN elements as zero.
+__device__ __forceinline__ half8_t finite_part(const half8_t& x) {
+  half8_t r;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) r[i] = __builtin_fabsf16(x[i]) < (_Float16)INFINITY ? x[i] : (_Float16)0.f;
+  return r;
+}
 // s / sqrt(D): exact for D = 64; an infinite score stays infinite.
 template <int D>
 __device__ __forceinline__ float score_of(float s, const EvalArgs& a) {
@@ -580,54 +587,70 @@ __global__ __launch_bounds__(64 * kEvalWaves) void prefill_eval_kernel(EvalArgs 
       __builtin_memcpy(reinterpret_cast<char*>(&x) + 8, &v2, 8);
       return x;
     };
-    for (int p = w; 32 * p < nmax; p += NW) {
-      auto load_chunks = [&](__amdgpu_buffer_rsrc_t r, half8_t (&x)[NCH]) {
-#pragma unroll
-        for (int k = 0; k < NCH; ++k) {
+    auto sums = [&](auto clean) {
+      constexpr bool CLEAN = decltype(clean)::value;
+      for (int p = w; 32 * p < nmax; p += NW) {
+        auto load_chunk = [&](__amdgpu_buffer_rsrc_t r, int k) {
+          half8_t x;
           const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, (uint32_t)32 * p * D * 2 + (lane + 64 * k) * 16, 0, 0);
-          __builtin_memcpy(&x[k], &v, 16);
+          __builtin_memcpy(&x, &v, 16);
+          return x;
+        };
+        auto load_chunks = [&](__amdgpu_buffer_rsrc_t r, half8_t (&x)[NCH]) {
+#pragma unroll
+          for (int k = 0; k < NCH; ++k) x[k] = load_chunk(r, k);
+        };
+        auto chunk = [&](int k) {
+          const int c = lane + 64 * k;
+          return reinterpret_cast<half8_t*>(vt + c / (D / 8) * VRS + c % (D / 8) * 16);
+        };
+        half8_t xh[NCH], xv[NCH];
+        if constexpr (D == 64 && !CLEAN) load_chunks(rvh, xh);
+        float wa[2][4], wk[2][4];
+        weights(p, wa, wk);
+        half8_t pa, ph, pl;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          pa[j] = (_Float16)wa[j >> 2][j & 3];
+          const float u = wk[j >> 2][j & 3] * kUp;
+          ph[j] = (_Float16)u;
+          pl[j] = (_Float16)(u - (float)ph[j]);
+          if constexpr (!CLEAN) wsum += wk[j >> 2][j & 3];
         }
-      };
-      auto chunk = [&](int k) {
-        const int c = lane + 64 * k;
-        return reinterpret_cast<half8_t*>(vt + c / (D / 8) * VRS + c % (D / 8) * 16);
-      };
-      half8_t xh[NCH], xv[NCH];
-      if constexpr (D == 64) load_chunks(rvh, xh);
-      float wa[2][4], wk[2][4];
-      weights(p, wa, wk);
-      half8_t pa, ph, pl;
+        if constexpr (D == 128 && !CLEAN) load_chunks(rvh, xh);
+        lds_sync_wave();  // the last tile's reads
+        if constexpr (CLEAN) {
+#pragma unroll 1
+          for (int k = 0; k < NCH; ++k) *chunk(k) = finite_part(load_chunk(rvh, k));
+        } else {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        pa[j] = (_Float16)wa[j >> 2][j & 3];
-        const float u = wk[j >> 2][j & 3] * kUp;
-        ph[j] = (_Float16)u;
-        pl[j] = (_Float16)(u - (float)ph[j]);
-        wsum += wk[j >> 2][j & 3];
+          for (int k = 0; k < NCH; ++k) *chunk(k) = xh[k];
+          load_chunks(rv, xv);
+        }
+        lds_sync_wave();
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+          const half8_t x = v_operand(dt);
+          ak[dt] = mfma16x32(x, ph, ak[dt]);
+          ak[dt] = mfma16x32(x, pl, ak[dt]);
+        }
+        if constexpr (CLEAN) {
+          lds_sync_wave();
+#pragma unroll 1
+          for (int k = 0; k < NCH; ++k) *chunk(k) = finite_part(minus(load_chunk(rv, k), load_chunk(rvh, k)));
+        } else {
+#pragma unroll
+          for (int k = 0; k < NCH; ++k) xv[k] = minus(xv[k], *chunk(k));  // r_v; the lane's own chunks of V_hat
+          lds_sync_wave();
+#pragma unroll
+          for (int k = 0; k < NCH; ++k) *chunk(k) = xv[k];
+        }
+        lds_sync_wave();
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) av[dt] = mfma16x32(v_operand(dt), pa, av[dt]);
       }
-      if constexpr (D == 128) load_chunks(rvh, xh);
-      lds_sync_wave();  // the last tile's reads
-#pragma unroll
-      for (int k = 0; k < NCH; ++k) *chunk(k) = xh[k];
-      load_chunks(rv, xv);
-      lds_sync_wave();
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        const half8_t x = v_operand(dt);
-        ak[dt] = mfma16x32(x, ph, ak[dt]);
-        ak[dt] = mfma16x32(x, pl, ak[dt]);
-      }
-#pragma unroll
-      for (int k = 0; k < NCH; ++k) xv[k] = minus(xv[k], *chunk(k));  // r_v; the lane's own chunks of V_hat
-      lds_sync_wave();
-#pragma unroll
-      for (int k = 0; k < NCH; ++k) *chunk(k) = xv[k];
-      lds_sync_wave();
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) av[dt] = mfma16x32(v_operand(dt), pa, av[dt]);
-    }
-    // an infinity or NaN in a token a row does not read must not reach it
-    // through a zero weight: such a wave sums its selected tokens alone
+    };
+    sums(std::false_type{});
     bool bad = false;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
@@ -636,9 +659,14 @@ __global__ __launch_bounds__(64 * kEvalWaves) void prefill_eval_kernel(EvalArgs 
         bad |= !(fabsf(av[dt][i]) < INFINITY);
         bad |= !(fabsf(ak[dt][i]) < INFINITY);
       }
-    if (__any(bad)) {
+    if (__builtin_expect(__any(bad), 0)) {
+      // An infinity or NaN in a token that a row does not read must not reach
+      // it through a zero weight: the sums are taken again without such
+      // elements, and the rows that read them add them afterwards.  The other
+      // rows keep the bits that they have without those elements.
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) av[dt] = ak[dt] = float4_t{0.f, 0.f, 0.f, 0.f};
+      sums(std::true_type{});
       for (int p = w; 32 * p < nmax; p += NW) {
         float wa[2][4], wk[2][4];
         weights(p, wa, wk);
@@ -656,8 +684,9 @@ __global__ __launch_bounds__(64 * kEvalWaves) void prefill_eval_kernel(EvalArgs 
 #pragma unroll
               for (int i = 0; i < 4; ++i) {
                 const _Float16 vhat = bits2half(a.vh[row + 16 * dt + i]);
-                av[dt][i] = fmaf(xa, (float)(_Float16)(bits2half(a.v[row + 16 * dt + i]) - vhat), av[dt][i]);
-                ak[dt][i] = fmaf(xk * kUp, (float)vhat, ak[dt][i]);
+                const float r = (float)(_Float16)(bits2half(a.v[row + 16 * dt + i]) - vhat), vf = (float)vhat;
+                if (!(fabsf(r) < INFINITY)) av[dt][i] = fmaf(xa, r, av[dt][i]);
+                if (!(fabsf(vf) < INFINITY)) ak[dt][i] = fmaf(xk * kUp, vf, ak[dt][i]);
               }
           }
       }
