@@ -326,14 +326,14 @@ __global__ __launch_bounds__(64 * kEvalWaves) void prefill_eval_kernel(EvalArgs 
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         vd2[i] = fmaf(-2.f, vo[i], vv2 + oo[i]);
-        near |= vd2[i] * 32.f < vv2 + oo[i];
+        near |= !(vd2[i] * 32.f >= vv2 + oo[i]);
       }
       if (__any(near)) {
-        // V_hat_j close to o (a row whose weight sits on one token): the
-        // expansion cancels, so those pairs take the difference itself
+        // V_hat_j close to o (a row whose weight sits on one token), or not
+        // finite: the expansion cancels, so those pairs take the difference itself
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          if (4 * g + i >= NC || !(vd2[i] * 32.f < vv2 + oo[i])) continue;
+          if (4 * g + i >= NC || vd2[i] * 32.f >= vv2 + oo[i]) continue;
           const uint32_t v_at = (uint32_t)min(tok, T - 1) * D * 2, o_at = (uint32_t)min(t0 + 4 * g + i, T - 1) * D * 2;
           float d2 = 0.f;
 #pragma unroll 1
@@ -376,8 +376,12 @@ __global__ __launch_bounds__(64 * kEvalWaves) void prefill_eval_kernel(EvalArgs 
           if constexpr (MODE == 0) x = vs + ks;
           if constexpr (MODE == 1) x = ks;
           if constexpr (MODE == 2) x = vs;
-          if constexpr (MODE == 3)
-            x = div_r(vs, vm[i], __builtin_amdgcn_rcpf(vm[i])) + div_r(ks, km[i], __builtin_amdgcn_rcpf(km[i]));
+          if constexpr (MODE == 3) {
+            // (over an infinite mean the rounded-off quotient itself: 0 for a
+            // finite score, which the Newton step would make NaN)
+            const float rv = __builtin_amdgcn_rcpf(vm[i]), rk = __builtin_amdgcn_rcpf(km[i]);
+            x = (vm[i] < INFINITY ? div_r(vs, vm[i], rv) : vs * rv) + (km[i] < INFINITY ? div_r(ks, km[i], rk) : ks * rk);
+          }
           sc[cl * stride + tok] = x;
         }
       }
