@@ -21,16 +21,20 @@
 //      cost less than gathering each row's own tokens.
 // Two work-groups cannot share a CU (the scores of 16 rows of 2048 tokens are
 // 131 KB of its 160 KB LDS), hence 16 waves.  Measured on a 2048-token prompt
-// of 32 query / 4 kv heads, D = 64, ratio 0.05: 553 us, against 5304 us for one
+// of 32 query / 4 kv heads, D = 64, ratio 0.05: 539 us, against 5324 us for one
 // work-group per (row, head) with scalar products, which read each row's tokens
-// from L2 twice (D = 128, 8 kv heads, 1024 tokens: 312 us).  Of the 580 us with
-// the clock of another run, launching and filling the CUs takes 26, step 1 58,
-// step 2 177, step 3 156 and step 4 163; steps 1, 2 and 4 are bound by the
-// loads' and lane exchanges' latency (four waves per SIMD, 45% VALU-busy),
-// step 3 by its compares.
+// from L2 twice (D = 128, 8 kv heads, 1024 tokens: 309 us, 1740 before).  Of the
+// 539 us (builds that end after a step) launching and filling the CUs takes at
+// most 20, step 1 56, step 2 147, step 3 158, step 4 127 and the output 31; steps
+// 1, 2 and 4 are bound by the loads' and lane exchanges' latency (four waves per
+// SIMD), step 3 by its compares.  At D = 128 the 128 VGPRs of a 16-wave
+// work-group do not hold step 4's tiles: 12 of the 646 instructions of its loop
+// are scratch accesses.  A prompt of 64 tokens takes one wave's latency through
+// the four steps, 20 us at D = 128 (24 with normalize), 28 for the scalar form.
 //
 // Every sum over a row's tokens is taken in an order that depends on the token
-// indices alone (tiles dealt to the 16 waves), so a row's result does not
+// indices alone (tiles dealt to the 16 waves), and infinities and NaN in tokens
+// that a row does not read are kept out of its sums, so a row's result does not
 // change with NC, the batch or the prompt's length after the row.
 #include <cmath>
 
@@ -108,10 +112,11 @@ __device__ __forceinline__ float score_of(float s, const EvalArgs& a) {
   if constexpr (D == 64) return s * 0.125f;
   return fabsf(s) < INFINITY ? div_r(s, a.sqrt_d, a.rcp_sqrt_d) : s;
 }
-// exp(x) for x <= 0 within 2 ulp: x log2(e) in two parts, the low one applied
-// to the base-2 exponential to first order.  Below -104, and for NaN, the
-// value at -104 (0 as a weight in fp16; a NaN score reaches the row through
-// its sum).
+// exp(x) for x <= 0 within 2 ulp: x log2(e) as an unevaluated sum of two floats
+// (Dekker's product with the FMA's exact remainder, log2(e) itself in two
+// floats), the low one applied to the base-2 exponential to first order.
+// Below -104, and for NaN, the value at -104 (0 as a weight in fp16; a NaN
+// score reaches the row through its sum).
 __device__ __forceinline__ float exp_neg(float x) {
   x = fmaxf(x, -104.f);
   const float ph = x * 1.44269502f;
@@ -119,7 +124,7 @@ __device__ __forceinline__ float exp_neg(float x) {
   const float e = __builtin_amdgcn_exp2f(ph);
   return fmaf(e, pl * 0.693147182f, e);
 }
-// Sums over the wave of an int and over the 16 lanes of a row of a float.
+// The sum and the union of bits over the wave, and the sum over the 16 lanes of a row.
 __device__ __forceinline__ int wave_isum(int v) {
   v += row_ror_i<8>(v);
   v += row_ror_i<4>(v);
@@ -129,6 +134,16 @@ __device__ __forceinline__ int wave_isum(int v) {
   v = (int)(p[0] + p[1]);
   const auto r = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
   return __builtin_amdgcn_readfirstlane((int)(r[0] + r[1]));
+}
+__device__ __forceinline__ uint32_t wave_or(uint32_t v) {
+  v |= (uint32_t)row_ror_i<8>((int)v);
+  v |= (uint32_t)row_ror_i<4>((int)v);
+  v |= (uint32_t)row_ror_i<2>((int)v);
+  v |= (uint32_t)row_ror_i<1>((int)v);
+  const auto p = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  v = p[0] | p[1];
+  const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)(r[0] | r[1]));
 }
 __device__ __forceinline__ float row16_sum(float v) {
   v += row_ror<8>(v);
@@ -147,6 +162,11 @@ __global__ __launch_bounds__(64 * kEvalWaves) void prefill_eval_kernel(EvalArgs 
   constexpr int CPP = eval_chunks(NC); // 512-token chunks per wave there
   constexpr int MW = 8 * CPP * WPC;    // 64-token words of a row's selection
   constexpr int VRS = 2 * D + 32;      // staged V row stride, bytes
+  // An expanded distance's terms are at most this multiple of its square (an error
+  // of 2^-24 of the terms is 2^-23 of the distance; the scores' dot products
+  // lose more).  Rows whose selection differs from 64-bit scores, of 500 000 rows:
+  // 4, against 6 for the differences alone and 8 with a multiple of 32.
+  constexpr float kCancel = 4.f;
   typedef short short4_t __attribute__((ext_vector_type(4)));
   typedef __attribute__((address_space(3))) short4_t lds_short4;
   typedef __attribute__((address_space(3))) char lds_char;
@@ -322,35 +342,42 @@ __global__ __launch_bounds__(64 * kEvalWaves) void prefill_eval_kernel(EvalArgs 
       if constexpr (MODE != 1) rvn = __builtin_amdgcn_sqrtf(diag(r2));
       const int tok = 16 * tile + c16;
       float vd2[4];
-      bool near = false;
+      uint32_t rows = 0;  // rows of the block with a token near their o
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         vd2[i] = fmaf(-2.f, vo[i], vv2 + oo[i]);
-        near |= !(vd2[i] * 32.f >= vv2 + oo[i]);
+        const uint64_t b = __ballot(4 * g + i < NC && !(vd2[i] * kCancel >= vv2 + oo[i]));
+#pragma unroll
+        for (int u = 0; u < 4; ++u) rows |= (b >> (16 * u) & 0xffff) != 0 ? 1u << (4 * u + i) : 0u;
       }
-      if (__any(near)) {
-        // V_hat_j close to o (a row whose weight sits on one token), or not
-        // finite: the expansion cancels, so those pairs take the difference itself
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if (4 * g + i >= NC || vd2[i] * 32.f >= vv2 + oo[i]) continue;
-          const uint32_t v_at = (uint32_t)min(tok, T - 1) * D * 2, o_at = (uint32_t)min(t0 + 4 * g + i, T - 1) * D * 2;
-          float d2 = 0.f;
+      // V_hat_j close to o (a row whose weight sits on few tokens), or not
+      // finite: the expansion cancels, so those pairs take the difference itself.
+      // The operands hold both sides: lane (c16, g) has token c16's dims
+      // 32 ks + 8 g .., and row r's come from lane (r, g).
 #pragma unroll 1
-          for (int d = 0; d < D; d += 8) {
-            half8_t y, z;
-            const auto yv = __builtin_amdgcn_raw_buffer_load_b128(rvh, v_at + 2 * d, 0, 0);
-            const auto zv = __builtin_amdgcn_raw_buffer_load_b128(ro, o_at + 2 * d, 0, 0);
-            __builtin_memcpy(&y, &yv, 16);
-            __builtin_memcpy(&z, &zv, 16);
+      while (rows != 0) {
+        const int r = __builtin_ctz(rows);
+        rows &= rows - 1;
+        float d2 = 0.f, one = 1.f;
+        asm("" : "+s"(one));  // (a visible 1 becomes a subtraction and two conversions)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-              const float df = (float)y[e] - (float)z[e];
-              d2 = fmaf(df, df, d2);
-            }
+        for (int ks = 0; ks < KS; ++ks) {
+          uint32_t ow[4];
+          __builtin_memcpy(ow, &of[ks], 16);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) ow[e] = (uint32_t)__builtin_amdgcn_ds_bpermute((r + 16 * g) * 4, (int)ow[e]);
+          half8_t o8;
+          __builtin_memcpy(&o8, ow, 16);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float df = fmaf((float)x.vh[ks][e], one, -(float)o8[e]);
+            d2 = fmaf(df, df, d2);
           }
-          vd2[i] = d2;
         }
+        d2 = col_sum(d2);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (r == 4 * g + i && !(vd2[i] * kCancel >= vv2 + oo[i])) vd2[i] = d2;
       }
       const float4_t mx = *reinterpret_cast<const float4_t*>(s_mx + 4 * g), den = *reinterpret_cast<const float4_t*>(s_den + 4 * g);
       float4_t vm, km;
@@ -475,7 +502,14 @@ __global__ __launch_bounds__(64 * kEvalWaves) void prefill_eval_kernel(EvalArgs 
     };
     uint32_t tau = 0u;
     bool cut = K == 0;  // exactly K keys are >= tau (K = 0: none is taken)
-    for (int bit = 31; bit >= 0; --bit) {
+    int bit = 31;
+    if constexpr (WPC == 1) {  // from the largest key's top bit (the scores of a short prompt's first rows are 0)
+      uint32_t any = 0u;
+#pragma unroll
+      for (int k = 0; k < 8 * CPP; ++k) any |= key[k];
+      bit = 31 - __builtin_clz(wave_or(any) | 1u);
+    }
+    for (; bit >= 0; --bit) {
       if (WPC == 1 && cut) break;  // a row of several waves passes every barrier
       const uint32_t cand = tau | (1u << bit);
       const int cnt = row_total(count_ge(cand));
