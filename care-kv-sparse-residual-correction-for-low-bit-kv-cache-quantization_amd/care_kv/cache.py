@@ -359,10 +359,12 @@ class CAREKVCache:
         """Forget a sequence slot (pages, metadata, residual slots)."""
         seq = range(self.n_seq)[operator.index(seq)]  # (a negative slot counts from the end)
         lib = _lib.load()
-        _lib.check(lib.carekv_reset_sequence(
-            self.valid.data_ptr(), self.has_meta.data_ptr(), self.k_slot.data_ptr(), self.v_slot.data_ptr(),
-            self.next_slot.data_ptr(), self.cfg.num_layers * self.cfg.num_kv_heads, self.n_seq, self.cfg.max_pages,
-            self.ncg, self.nvb, seq, _lib.stream_ptr(self.device)), "carekv_reset_sequence")
+        dev = self.valid.device
+        with torch.cuda.device(dev):  # whatever device the caller has current, as the tensors' own operations
+            _lib.check(lib.carekv_reset_sequence(
+                self.valid.data_ptr(), self.has_meta.data_ptr(), self.k_slot.data_ptr(), self.v_slot.data_ptr(),
+                self.next_slot.data_ptr(), self.cfg.num_layers * self.cfg.num_kv_heads, self.n_seq, self.cfg.max_pages,
+                self.ncg, self.nvb, seq, _lib.stream_ptr(dev)), "carekv_reset_sequence")
         self._freed.pop((seq, 0), None)
         self._freed.pop((seq, 1), None)
         self.next_page[:, :, seq] = 0
