@@ -270,6 +270,8 @@ def decode_attention(cache: CAREKVCache, layer: int, q: torch.Tensor, seqs: Opti
     B, Hq, D = q.shape
     assert D == cfg.head_dim and Hq == cfg.num_heads
     seqs = list(range(B)) if seqs is None else list(seqs)
+    if len(seqs) < B:  # the kernels read a sequence slot and a page count per row of q
+        raise ValueError(f"decode_attention: {B} rows of q for {len(seqs)} sequence slots")
     if knobs is None:
         knobs = resolve_read_knobs(cfg, layer)
     q = q.to(torch.float16).contiguous()

@@ -1,5 +1,5 @@
-"""``CAREKVCache.append``'s host bookkeeping without a device: a destination is
-made for every row that the kernel is told to read."""
+"""The host tables of ``CAREKVCache.append`` and ``decode_attention`` without a
+device: an entry is made for every row that the kernels are told to read."""
 import numpy as np
 import pytest
 import torch
@@ -50,3 +50,10 @@ def test_a_destination_for_every_row(cache):
         assert cache.lib.n_rows == 2 * B == len(cache.tables[-1])
         assert cache.tables[-1][:, 0].tolist() == [s for s in (seqs or range(B)) for _ in range(2)]
         assert cache.tables[-1][:, 1].tolist() == [0, 1] * B
+
+
+def test_decode_rows_without_a_slot_are_refused(cache):
+    q = torch.zeros(3, 4, 64, dtype=torch.float16)
+    for seqs in ([], [0], [0, 2]):
+        with pytest.raises(ValueError):
+            care_kv.decode_attention(cache, 0, q, seqs=seqs)
