@@ -707,8 +707,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
 // rank order, a butterfly per 64 pages, then the four totals in page order),
 // the k-th largest key comes from a binary search over its 31 bits, and ties
 // at it are taken in candidate order, so the (M, L), masks and diag lists are
-// the same bits.  The search ends as soon as exactly k keys lie above its
-// bound (usually after half the bits) and starts at the largest key's top bit.
+// the same bits.  The search starts at the largest key's top bit and ends once
+// exactly k keys lie above its bound (usually after half the bits).
 // The joint or separate policy, no adaptive_score, correction on, the moments'
 // K score.
 template <int D, bool K1>
@@ -1010,13 +1010,21 @@ __global__ __launch_bounds__(256) void decode_select_wave_kernel(carekv_arena A,
     top = row4_max_i(max(top, row_ror_i<2>(top)));
     top = pair32_max_i(pair16_max_i(max(top, row_ror_i<1>(top))));
     top = __builtin_amdgcn_readfirstlane(top);
+    // four bits between tests for an exact count: a test a bit puts the count's
+    // latency and a branch on every step, and the slowest column of a launch
+    // has ties that no bit ends (30 x 8 rows of 14 pages: that column 4.5 us,
+    // 2.4 without tests)
     uint32_t tau = 0u;
-    for (int bit = 31 - __builtin_clz(top | 1); bit >= 0; --bit) {
-      const uint32_t t = tau | (1u << bit);
-      const int n = count_ge((int)t, useK, useV);
-      if (n < k) continue;
-      tau = t;
-      if (n == k) {  // every key at or above tau, no tie to rank
+    int at = INT_MAX;  // keys at or above tau
+    for (int bit = (31 - __builtin_clz(top | 1)) | 3; bit >= 0; bit -= 4) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const uint32_t t = tau | (1u << (bit - u) & 0x7fffffffu);
+        const int n = count_ge((int)t, useK, useV);
+        at = n >= k ? n : at;
+        tau = n >= k ? t : tau;
+      }
+      if (at == k) {  // every key at or above tau, no tie to rank
         r.tau = tau;
         return r;
       }
