@@ -277,6 +277,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
 
   // ---- q sketches q_cg P (fp32, attention.py:722) for the proxy
   const int skd = A.sketch_dim;
+  // sketch rows of whole 16-byte chunks, where the caller's table is aligned to them
+  const bool wide = (skd & 7) == 0 && (reinterpret_cast<uintptr_t>(A.k_sketch) & 15) == 0;
   if constexpr (PX) {
     const uint16_t* qg = a.q + ((long)b * a.Hq + kvh * GQ + qq) * D;
     if (a.pf) {  // prefill rows: the column's (row, head); a padding column sketches zero
@@ -335,7 +337,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
         const uint16_t* ks = A.k_sketch + (pg * NCG + cg) * skd;
         const float* qs = s_qs + cg * 68;
         float dot = 0.f;
-        if ((skd & 7) == 0) {
+        if (wide) {
 #pragma unroll 4
           for (int j = 0; j < skd; j += 8) {
             const uint4 v = *reinterpret_cast<const uint4*>(ks + j);
