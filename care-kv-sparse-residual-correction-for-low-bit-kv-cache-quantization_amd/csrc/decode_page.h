@@ -639,6 +639,18 @@ __device__ __forceinline__ float row4_max(float v) {
   v = fmaxf(v, row_ror<4>(v));
   return fmaxf(v, row_ror<8>(v));
 }
+// Sum over the 16 lanes of a row.
+__device__ __forceinline__ float row16_sum(float v) {
+  v += row_ror<8>(v);
+  v += row_ror<4>(v);
+  v += row_ror<2>(v);
+  return v + row_ror<1>(v);
+}
+// m[c16][c16] of a 16x16 product (lane (c16, g) holds m[4 g + i][c16]) in every lane of its column.
+__device__ __forceinline__ float diag16(const float4_t& m, int c16, int g) {
+  const float lo = c16 & 1 ? m[1] : m[0], hi = c16 & 1 ? m[3] : m[2];
+  return col_sum(c16 >> 2 == g ? (c16 & 2 ? hi : lo) : 0.f);
+}
 
 // Max / min reductions on integers: one DPP or lane-swap op per step, where
 // the float max needs its inputs canonicalised first.

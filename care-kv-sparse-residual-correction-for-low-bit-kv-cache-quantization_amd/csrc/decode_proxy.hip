@@ -43,14 +43,6 @@
 
 namespace carekv {
 
-// Sum over the 16 lanes of a row.
-__device__ __forceinline__ float row16_sum(float v) {
-  v += row_ror<8>(v);
-  v += row_ror<4>(v);
-  v += row_ror<2>(v);
-  return v + row_ror<1>(v);
-}
-
 // NG: groups of four queries whose operands a wave holds.
 template <int D, int BITS, int SM, int NG, bool PF = false>
 __global__ __launch_bounds__(256) void decode_proxy_kernel(carekv_arena A, DecodeArgs a) {
@@ -216,9 +208,7 @@ __global__ __launch_bounds__(256) void decode_proxy_kernel(carekv_arena A, Decod
     float4_t v2{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) v2 = mfma16x32(vb[ks], vb[ks], v2);
-    // token ln's norm: the diagonal, held by the lane with lj = ln / 4
-    const float dlo = ln & 1 ? v2[1] : v2[0], dhi = ln & 1 ? v2[3] : v2[2];
-    const float vv = col_sum(ln >> 2 == lj ? (ln & 2 ? dhi : dlo) : 0.f);
+    const float vv = diag16(v2, ln, lj);  // token ln's norm
 
 #pragma unroll
     for (int k = 0; k < NG; ++k) {

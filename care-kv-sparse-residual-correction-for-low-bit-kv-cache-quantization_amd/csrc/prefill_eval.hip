@@ -124,7 +124,7 @@ __device__ __forceinline__ float exp_neg(float x) {
   const float e = __builtin_amdgcn_exp2f(ph);
   return fmaf(e, pl * 0.693147182f, e);
 }
-// The sum and the union of bits over the wave, and the sum over the 16 lanes of a row.
+// The sum and the union of bits over the wave.
 __device__ __forceinline__ int wave_isum(int v) {
   v += row_ror_i<8>(v);
   v += row_ror_i<4>(v);
@@ -144,13 +144,6 @@ __device__ __forceinline__ uint32_t wave_or(uint32_t v) {
   v = p[0] | p[1];
   const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
   return (uint32_t)__builtin_amdgcn_readfirstlane((int)(r[0] | r[1]));
-}
-__device__ __forceinline__ float row16_sum(float v) {
-  v += row_ror<8>(v);
-  v += row_ror<4>(v);
-  v += row_ror<2>(v);
-  v += row_ror<1>(v);
-  return v;
 }
 
 template <int D, int NC>
@@ -331,15 +324,10 @@ __global__ __launch_bounds__(64 * kEvalWaves) void prefill_eval_kernel(EvalArgs 
           r2 = mfma16x32(r, r, r2);
         }
       }
-      // the squared norms of token c16: the diagonals of V_hat V_hat^T and
-      // r_v r_v^T, held by the lanes with g = c16 / 4
-      auto diag = [&](const float4_t& m) {
-        const float lo = c16 & 1 ? m[1] : m[0], hi = c16 & 1 ? m[3] : m[2];
-        return col_sum(c16 >> 2 == g ? (c16 & 2 ? hi : lo) : 0.f);
-      };
-      const float vv2 = diag(v2);
+      // the squared norms of token c16: the diagonals of V_hat V_hat^T and r_v r_v^T
+      const float vv2 = diag16(v2, c16, g);
       float rvn = 0.f;
-      if constexpr (MODE != 1) rvn = __builtin_amdgcn_sqrtf(diag(r2));
+      if constexpr (MODE != 1) rvn = __builtin_amdgcn_sqrtf(diag16(r2, c16, g));
       const int tok = 16 * tile + c16;
       float vd2[4];
       uint32_t rows = 0;  // rows of the block with a token near their o
