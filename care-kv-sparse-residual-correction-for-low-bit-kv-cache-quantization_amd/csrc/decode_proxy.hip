@@ -23,13 +23,13 @@
 // finite, the pair takes the differences themselves, so that the distances keep
 // the differences' error against 64 bits (D = 128, rms: V around zero 4.7e-8,
 // differences 4.8e-8; around one deviation 5.3e-8 both, 6.5e-8 where it may
-// lose half; around 3.5 deviations 7.6e-8 both, 4.3e-7 where it may lose 31/32).  A page of 4 queries costs about
-// 200 VALU operations and 8 MFMAs; the differences alone took 384 VALU and 128
-// LDS reads.  A page's loads are issued while the page before it
-// is worked on, and the split statistics are read by lanes side by side (a thread
-// per query walked them before, two memory round trips a split).  Measured at
-// 8 sequences x 8 kv heads x 8185 tokens, INT4, D = 128, 4 queries:
-// 31.3 us, 57.7 us before.
+// lose half; around 3.5 deviations 7.6e-8 both, 4.3e-7 where it may lose
+// 31/32).  A page of 4 queries costs about 200 VALU operations and 8 MFMAs; the
+// differences alone took 384 VALU and 128 LDS reads.  A page's loads are issued
+// while the page before it is worked on, and the split statistics are read by
+// lanes side by side (a thread per query walked them before, two memory round
+// trips a split).  Measured at 8 sequences x 8 kv heads x 8185 tokens, INT4, D =
+// 128, 4 queries: 31.2 us, 56.8 us before.
 //
 // PF (prefill rows, the per-(head, row) router of correction_impl=cached,
 // layer.py:573-640): a is the reference's fp16 attention weight of the row

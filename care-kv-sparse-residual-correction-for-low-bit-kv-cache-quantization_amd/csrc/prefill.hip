@@ -10,14 +10,15 @@
 // K and V tiles of 32 tokens are staged in LDS (double buffered, one barrier per
 // tile; the next tile's global loads are in flight while the current one is
 // used); at D = 128, 160 VGPRs and 35 KB of LDS, three work-groups share a CU.
-// 48 queries a wave (218 VGPRs, two work-groups) measured the same (4 x 40 heads, T =
-// 8192: 2912 us against 2917; 8 x 32 / 8 heads, T = 3000: 692 against 686).
+// 48 queries a wave (218 VGPRs, two work-groups) measured the same (4 x 40
+// heads, T = 8192: 2912 us against 2917; 8 x 32 / 8 heads, T = 3000: 692 against
+// 686).
 //   * S^T = K_hat Q^T: A = K tile rows (one 16-byte LDS read per lane and
 //     32-dim step), B = Q^T held in registers; lane l receives the scores of
 //     tokens 16tt + 4(l/16) + i for query l % 16 of a 16-query sub-block;
 //   * the online softmax runs per query column in fp32 on base-2 logits
 //     (scores scaled by log2(e)/sqrt(D) after the fp32 product, as the
-//     reference divides the fp32 product by sqrt(D));
+//     reference divides the fp32 product by sqrt(D)).
 //     Each lane compares its own 8 scores with the column's running maximum;
 //     only where one is larger are they reduced over the lane groups, the sums
 //     rescaled and the maximum moved.  Columns that keep theirs are multiplied
