@@ -23,14 +23,14 @@
 // 131 KB of its 160 KB LDS), hence 16 waves.  Measured on a 2048-token prompt
 // of 32 query / 4 kv heads, D = 64, ratio 0.05: 539 us, against 5324 us for one
 // work-group per (row, head) with scalar products, which read each row's tokens
-// from L2 twice (D = 128, 8 kv heads, 1024 tokens: 309 us, 1740 before).  Of the
+// from L2 twice (D = 128, 8 kv heads, 1024 tokens: 305 us, 1720 before).  Of the
 // 539 us (builds that end after a step) launching and filling the CUs takes at
 // most 20, step 1 56, step 2 147, step 3 158, step 4 127 and the output 31; steps
 // 1, 2 and 4 are bound by the loads' and lane exchanges' latency (four waves per
 // SIMD), step 3 by its compares.  At D = 128 the 128 VGPRs of a 16-wave
 // work-group do not hold step 4's tiles: 12 of the 646 instructions of its loop
 // are scratch accesses.  A prompt of 64 tokens takes one wave's latency through
-// the four steps, 20 us at D = 128 (24 with normalize), 28 for the scalar form.
+// the four steps, 19 us at D = 128 (21 with normalize), 28 for the scalar form.
 //
 // Every sum over a row's tokens is taken in an order that depends on the token
 // indices alone (tiles dealt to the 16 waves), and infinities and NaN in tokens
@@ -722,6 +722,7 @@ __global__ __launch_bounds__(64 * kEvalWaves) void prefill_eval_kernel(EvalArgs 
   }
   // ---- the waves' sums in wave order, and the output
   constexpr int NO = D * NC / (64 * NW) > 0 ? D * NC / (64 * NW) : 1;  // outputs a thread forms
+  const int nact = min(NW, (nmax + 31) / 32);  // waves that had tokens; the others' sums are 0
   float tv[NO], tk[NO];
 #pragma unroll
   for (int half = 0; half < 2; ++half) {
@@ -731,18 +732,21 @@ __global__ __launch_bounds__(64 * kEvalWaves) void prefill_eval_kernel(EvalArgs 
       continue;
     }
     __syncthreads();
+    if (w < nact) {
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
+      for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        sc[(w * D + 16 * dt + 4 * g + i) * 17 + c16] = half ? ak[dt][i] : av[dt][i];
+        for (int i = 0; i < 4; ++i)
+          sc[(w * D + 16 * dt + 4 * g + i) * 17 + c16] = half ? ak[dt][i] : av[dt][i];
+    }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < NO; ++k) {
       const int id = tid + 64 * NW * k, cl = id / D, d = id % D;
       float x = 0.f;
       if (cl < NC)
-        for (int u = 0; u < NW; ++u) x += sc[(u * D + d) * 17 + cl];
+#pragma unroll 4
+        for (int u = 0; u < nact; ++u) x += sc[(u * D + d) * 17 + cl];
       if (half) tk[k] = x * kDown;
       else tv[k] = x;
     }
@@ -756,7 +760,7 @@ __global__ __launch_bounds__(64 * kEvalWaves) void prefill_eval_kernel(EvalArgs 
     float dk = 0.f;
     if (a.kind != 2 && some) {
       float ws = 0.f;
-      for (int u = 0; u < NW; ++u) ws += s_w[u][cl];
+      for (int u = 0; u < nact; ++u) ws += s_w[u][cl];
       dk = fmaf(-ws, o, tk[k]);
     }
     const float dv = a.kind == 1 ? 0.f : tv[k];
